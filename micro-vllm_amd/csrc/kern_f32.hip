@@ -5,23 +5,17 @@
 //
 // C[r, o] = sum_k X[r, k] * W[o, k] with f32 products and f32 sums (the reference's
 // matmul_f32 in another summation order).  Work item = (expert, block of up to 16 * MT
-// rows) x (block of columns).  Each wave computes MT row tiles x 2 column tiles of 16
-// (dual: the gate and the up rows of the same 16 columns, then the activation; single:
-// two adjacent tiles) and streams K in blocks of 16: lane (t, q) loads 16 bytes of row t
-// of each operand at K offset 4 q, and MFMA step s takes element s of them, so the four
-// steps of a block cover its 16 K indices once.  Waves are independent (no LDS, no
-// barrier); loads of the next block are issued before the current one is multiplied.
+// rows) x (block of columns).  Lane (t, q) loads 16 bytes of row t of each operand at K
+// offset 4 q, and MFMA step s takes element s of them, so the four steps of a 16-wide K
+// block cover its K indices once.
 // I8: a linear on QuantMat's int8 rows (fmt 8; quant::matmul_int8_row,
-// src/quant/quant.cpp:255-268): lane (t, q) loads the 4 codes of row t at K offset 4 q,
-// each converts exactly to f32, and the row's f32 scale multiplies the finished sum once,
-// as the reference does.
+// src/quant/quant.cpp:255-268): each code converts exactly to f32, and the row's f32 scale
+// multiplies the finished sum once, as the reference does.
 #include "mfma_common.h"
 
 #include <algorithm>
 
 namespace mvllm_hip {
-
-constexpr int kF32Waves = 4;
 
 struct F32Item {
     int a, r0, nrow, pad;
@@ -36,23 +30,44 @@ struct F32Args {
     const float *in;        // input rows [*][K]
     const int *in_rows;     // compact row -> input row (null: identity)
     float *out;             // output rows [rcap][O]
+    float *out2;            // the second half of K's sums when K is split (ksl = 1)
     int mi;                 // single: which matrix of the expert (2 = down; 0 = a linear)
-    int nbn, K, O;
+    int n_items, ksl;       // items; log2 of the K splits across workgroups (0 or 1)
+    int n_tasks, K, O;
     int act;
     float act_a, act_b;
 };
 
-template <bool DUAL, int MT, bool I8 = false>
-__global__ __launch_bounds__(64 * kF32Waves) void k_f32mm(F32Args A) {
-    static_assert(!(I8 && DUAL), "int8 rows: single projections only");
-    const int item = blockIdx.x / A.nbn;
-    const int nb = blockIdx.x - item * A.nbn;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int lane = threadIdx.x & 63, t = lane & 15, q = lane >> 4;
+// How the int8 codes of one row reach a lane: none (f32 rows), 4 codes of each 16-wide K
+// block, or 16 codes of each 64-wide one (K % 64 == 0 and 16-byte aligned rows).
+enum : int { kRowsF32 = 0, kRowsI8x4 = 1, kRowsI8x16 = 2 };
+
+// With few rows the weights' stream is the bound, and a wave per column tile walking all of
+// K left most of the chip idle (7168 x 384 at one row: 3 workgroups, 221 us for 11 MB).  So
+// the W waves of a workgroup split K of the same NT tiles of 16 weight rows and meet once
+// in LDS, where one thread per output adds the W partial sums in wave order (a fixed order:
+// equal inputs give equal bits; chains W times shorter, so no less exact).  Dual: the gate
+// and the up rows of 16 columns (NT = 2) or of 8 columns, side by side in one tile (NT = 1).
+// Two groups of U K blocks per operand are in flight per wave; loads past the wave's range
+// repeat its last block and are not multiplied.  Against the wave-per-tile kernel: the f32
+// expert of 7168 x 2048 at one row 300 -> 54 us per call (176 MB, 3.2 TB/s with the
+// combine), int8 7168 x 7168 167 -> 22 us, f32 7168 x 7168 at 61 rows 526 -> 103 us.
+template <bool DUAL, int MT, int NT, int WK, int W>
+__global__ __launch_bounds__(64 * W) void k_f32mm_rows(F32Args A) {
+    static_assert(!(WK && DUAL), "int8 rows: single projections only");
+    constexpr int KBW = WK == kRowsI8x16 ? 64 : 16;  // K indices of a block
+    constexpr int XV = KBW / 16;                     // float4 of an input row per lane and block
+    constexpr int U = WK == kRowsI8x16 ? (MT == 1 ? 2 : 1) : (MT == 1 ? 4 : 2);
+    __shared__ float red[W][MT * NT * 256];
+    const int task = xcd_task(blockIdx.x, A.n_tasks);
+    const int cs = task / A.n_items, item = task - cs * A.n_items;
+    const int ks = cs & ((1 << A.ksl) - 1), cb = cs >> A.ksl;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, t = lane & 15, q = lane >> 4;
     const int K = A.K, O = A.O;
-    const int col0 = DUAL ? (nb * kF32Waves + wave) * 16 : (nb * kF32Waves + wave) * 32;
-    if (col0 >= O)
-        return;  // past the last column tile (waves share nothing: no barrier below)
+    constexpr int CW = DUAL ? 8 * NT : 16 * NT;  // output columns of a workgroup
+    const int col0 = cb * CW;
     F32Item it;
     if (A.items) {
         it = A.items[item];
@@ -63,97 +78,134 @@ __global__ __launch_bounds__(64 * kF32Waves) void k_f32mm(F32Args A) {
     }
     const ExpertWork &ew = A.items ? A.ew[it.a] : A.ew1;
     const int jbase = ew.row0 + it.r0;
-    // operand row pointers of this lane: MT input rows, two weight rows
     const float4 *xr[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int r = min(mt * 16 + t, it.nrow - 1);  // rows past the item repeat the last
         const int src = A.in_rows ? A.in_rows[jbase + r] : jbase + r;
-        xr[mt] = reinterpret_cast<const float4 *>(A.in + (size_t)src * K) + q;
+        xr[mt] = reinterpret_cast<const float4 *>(A.in + (size_t)src * K) + XV * q;
     }
-    const float4 *wr[2];
-    const int *wr8[2];  // I8: 4 codes of row t at K offset 4 q of each 16-wide block
+    const char *wr[NT];
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const int row = DUAL ? col0 + t : col0 + 16 * m + t;
-        if constexpr (I8) {
-            const int8_t *w = static_cast<const int8_t *>(ew.w[A.mi]);
-            wr8[m] = reinterpret_cast<const int *>(w + (size_t)row * K) + q;
-        } else {
-            const float *w = static_cast<const float *>(ew.w[DUAL ? m : A.mi]);
-            wr[m] = reinterpret_cast<const float4 *>(w + (size_t)row * K) + q;
-        }
+    for (int m = 0; m < NT; ++m) {
+        const int row = DUAL ? col0 + (NT == 1 ? t & 7 : t) : col0 + 16 * m + t;
+        const char *w = static_cast<const char *>(ew.w[DUAL ? (NT == 1 ? t >> 3 : m) : A.mi]);
+        wr[m] = w + (size_t)row * (size_t)K * (WK ? 1 : 4) + (WK == kRowsI8x4 ? 4 : 16) * q;
     }
-    f4v acc[MT][2];
+    f4v acc[MT][NT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-        acc[mt][0] = acc[mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
-    const int nkb = K >> 4;  // 16-wide K blocks; a block is 4 float4 per row
-    float4 xa[2][MT], wb[2][2];
-    int wq[2][2];  // I8: raw codes
-    auto load = [&](int kb, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-            xa[buf][mt] = xr[mt][4 * kb];
+        for (int m = 0; m < NT; ++m)
+            acc[mt][m] = f4v{0.f, 0.f, 0.f, 0.f};
+    // this wave's K blocks [kb0, kb1)
+    const unsigned nkb = (unsigned)(K / KBW), part = (unsigned)(ks * W + wave);
+    constexpr int LW = W == 16 ? 4 : W == 8 ? 3 : 2;
+    const int kb0 = (int)(nkb * part >> (LW + A.ksl));
+    const int kb1 = (int)(nkb * (part + 1) >> (LW + A.ksl));
+    const int klast = max(kb1 - 1, 0);
+    struct Buf {
+        float4 x[U][MT][XV];
+        u32x4 w[U][NT];  // kRowsI8x4: word 0 only
+    };
+    auto load = [&] __attribute__((always_inline)) (Buf &b, int kb) {
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            if constexpr (I8)
-                wq[buf][m] = wr8[m][4 * kb];
-            else
-                wb[buf][m] = wr[m][4 * kb];
+        for (int u = 0; u < U; ++u) {
+            const int k = min(kb + u, klast);
+#pragma unroll
+            for (int m = 0; m < NT; ++m) {
+                const char *p = wr[m] + (size_t)k * (WK ? KBW : 64);
+                if constexpr (WK == kRowsI8x4)
+                    b.w[u][m].x = *reinterpret_cast<const uint32_t *>(p);
+                else
+                    b.w[u][m] = *reinterpret_cast<const u32x4 *>(p);
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int v = 0; v < XV; ++v)
+                    b.x[u][mt][v] = xr[mt][(size_t)k * (KBW / 4) + v];
         }
     };
-    auto mma = [&](int buf) __attribute__((always_inline)) {
+    auto mma = [&] __attribute__((always_inline)) (const Buf &b, int u) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int v = 0; v < XV; ++v)
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                float4 b;
-                if constexpr (I8) {
-                    const int v = wq[buf][m];
-                    b = float4{(float)(int8_t)(v & 0xff), (float)(int8_t)((v >> 8) & 0xff),
-                               (float)(int8_t)((v >> 16) & 0xff), (float)(int8_t)(v >> 24)};
-                } else {
-                    b = wb[buf][m];
+            for (int m = 0; m < NT; ++m) {
+                float w[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (WK == kRowsF32)
+                        w[e] = __uint_as_float(b.w[u][m][e]);
+                    else
+                        w[e] = (float)(int8_t)(b.w[u][m][v] >> (8 * e));
                 }
-                const float4 a = xa[buf][mt];
-                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc[mt][m], 0, 0, 0);
-                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc[mt][m], 0, 0, 0);
-                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc[mt][m], 0, 0, 0);
-                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc[mt][m], 0, 0, 0);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const float4 x = b.x[u][mt][v];
+                    acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, w[0], acc[mt][m], 0, 0, 0);
+                    acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, w[1], acc[mt][m], 0, 0, 0);
+                    acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, w[2], acc[mt][m], 0, 0, 0);
+                    acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, w[3], acc[mt][m], 0, 0, 0);
+                }
             }
     };
-    // two blocks in flight: block kb + 1 loads while block kb multiplies (past the end:
-    // the last block again, never consumed)
-    load(0, 0);
-    for (int kb = 0; kb < nkb; kb += 2) {
-        load(min(kb + 1, nkb - 1), 1);
-        mma(0);
-        if (kb + 1 >= nkb)
-            break;
-        load(min(kb + 2, nkb - 1), 0);
-        mma(1);
+    // groups of U blocks, two buffers; the pair loop has no exit between its two halves, and
+    // the last group(s) run after it with a uniform test per block
+    Buf b0, b1;
+    int kb = kb0;
+    load(b0, kb);
+    for (; kb + 2 * U <= kb1; kb += 2 * U) {
+        load(b1, kb + U);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            mma(b0, u);
+        load(b0, kb + 2 * U);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            mma(b1, u);
     }
-    // C[4 q + i][t] of row tile mt and column tile m
+    load(b1, kb + U);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (kb + u < kb1)
+            mma(b0, u);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (kb + U + u < kb1)
+            mma(b1, u);
+    // C[4 q + i][t] of row tile mt and tile m -> LDS, then the W partial sums in wave order
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = mt * 16 + 4 * q + i;
-            if (r >= it.nrow)
-                continue;
-            float *dst = A.out + (size_t)(jbase + r) * O;
-            if constexpr (DUAL) {
-                dst[col0 + t] = mf_act(A.act, acc[mt][0][i], acc[mt][1][i], A.act_a, A.act_b);
-            } else if constexpr (I8) {
-                const float *sc = static_cast<const float *>(ew.s[A.mi]);
-                dst[col0 + t] = acc[mt][0][i] * sc[col0 + t];
-                dst[col0 + 16 + t] = acc[mt][1][i] * sc[col0 + 16 + t];
-            } else {
-                dst[col0 + t] = acc[mt][0][i];
-                dst[col0 + 16 + t] = acc[mt][1][i];
-            }
-        }
+        for (int m = 0; m < NT; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                red[wave][(mt * NT + m) * 256 + i * 64 + lane] = acc[mt][m][i];
+    __syncthreads();
+    auto sum = [&] __attribute__((always_inline)) (int at) {
+        float v = red[0][at];
+#pragma unroll
+        for (int w = 1; w < W; ++w)
+            v += red[w][at];
+        return v;
+    };
+    for (int e = tid; e < MT * (DUAL ? 1 : NT) * 256; e += 64 * W) {
+        const int tile = e >> 8, pos = e & 255;
+        const int mt = DUAL ? tile : tile / NT, m = DUAL ? 0 : tile - mt * NT;
+        const int r = mt * 16 + 4 * ((pos >> 4) & 3) + (pos >> 6);
+        const int col = col0 + 16 * m + (pos & 15);
+        if (r >= it.nrow || (DUAL && NT == 1 && (pos & 8)))
+            continue;
+        float *dst = (ks ? A.out2 : A.out) + (size_t)(jbase + r) * O + col;
+        if constexpr (DUAL)
+            *dst = mf_act(A.act, sum(NT * tile * 256 + pos),
+                          sum(NT == 1 ? e + 8 : (2 * tile + 1) * 256 + pos), A.act_a, A.act_b);
+        else if constexpr (WK != kRowsF32)
+            *dst = sum(e) * static_cast<const float *>(ew.s[A.mi])[col];
+        else
+            *dst = sum(e);
+    }
 }
 
 bool f32mm_fits(bool dual, int K, int O) {
@@ -163,9 +215,9 @@ bool f32mm_fits(bool dual, int K, int O) {
 hipError_t launch_f32mm(bool dual, int mt, const ExpertWork *ew, const void *items, int n_items,
                         const ExpertWork *ew1, int nrows_all, const float *in,
                         const int *in_rows, float *out, int mi, int K, int O, int act,
-                        float act_a, float act_b, hipStream_t st, bool i8) {
+                        float act_a, float act_b, hipStream_t st, bool i8, float *out2) {
     if (!f32mm_fits(dual, K, O) || (mt != 1 && mt != 2 && mt != 4) || (!items && !ew1) ||
-        (i8 && dual))
+        (i8 && (dual || out2)) || (dual && out2))
         return hipErrorInvalidValue;
     F32Args a{};
     a.ew = ew;
@@ -176,30 +228,60 @@ hipError_t launch_f32mm(bool dual, int mt, const ExpertWork *ew, const void *ite
     a.in = in;
     a.in_rows = in_rows;
     a.out = out;
+    a.out2 = out2;
+    a.ksl = out2 ? 1 : 0;
     a.mi = mi;
     a.K = K;
     a.O = O;
     a.act = act;
     a.act_a = act_a;
     a.act_b = act_b;
-    const int cols_wg = (dual ? 16 : 32) * kF32Waves;
-    a.nbn = (O + cols_wg - 1) / cols_wg;
     if (!items)
         n_items = (nrows_all + 16 * mt - 1) / (16 * mt);
     if (n_items <= 0)
         return hipSuccess;
-    const dim3 grid((unsigned)(n_items * a.nbn)), block(64 * kF32Waves);
-#define MVLLM_F32(D, M) hipLaunchKernelGGL((k_f32mm<D, M>), grid, block, 0, st, a)
-#define MVLLM_I8(M) hipLaunchKernelGGL((k_f32mm<false, M, true>), grid, block, 0, st, a)
-    if (i8) {
-        if (mt == 1) MVLLM_I8(1); else if (mt == 2) MVLLM_I8(2); else MVLLM_I8(4);
-    } else if (dual) {
-        if (mt == 1) MVLLM_F32(true, 1); else if (mt == 2) MVLLM_F32(true, 2); else MVLLM_F32(true, 4);
-    } else {
-        if (mt == 1) MVLLM_F32(false, 1); else if (mt == 2) MVLLM_F32(false, 2); else MVLLM_F32(false, 4);
-    }
+    a.n_items = n_items;
+    const bool wide8 = i8 && K % 64 == 0 && ew1 && (reinterpret_cast<uintptr_t>(ew1->w[mi]) & 15) == 0;
+    // Two tiles a wave read the input rows once for twice the weights; one tile a wave gives
+    // twice the workgroups.  Two from 448 one-tile tasks on (the 256 CUs then have about a
+    // workgroup each): int8 7168 x 7168 at 16 rows 28 us against 42 us with one tile, f32
+    // 7168 x 7168 at 61 rows 103 against 154 us; below, one: the f32 expert of 7168 x 2048 at
+    // one row 54 against 77 us, 2048 x 2048 at 8 rows 11 against 22 us.  Sixteen waves split a
+    // long K of a launch that leaves CUs to spare (the same expert 54 against 57 us with
+    // eight, int8 7168 x 7168 22 against 25 us); shorter rows pay more for the larger
+    // workgroup's start than they gain (2048 x 2048 14 against 11 us).
+    const long long t1 = (long long)n_items * (O / (dual ? 8 : 16)) << a.ksl;
+    const int nt = t1 >= 448 ? 2 : 1;
+    const int w = mt == 1 && K >= 4096 && t1 / nt <= 256 ? 16 : 8;
+    a.n_tasks = (int)(t1 / nt);
+    const dim3 grid((unsigned)a.n_tasks), block((unsigned)(64 * w));
+#define MVLLM_F32(D, M, N, I, W_) \
+    hipLaunchKernelGGL((k_f32mm_rows<D, M, N, I, W_>), grid, block, 0, st, a)
+#define MVLLM_F32_MT(D, N, I)                                     \
+    do {                                                          \
+        if (mt == 1 && w == 16) MVLLM_F32(D, 1, N, I, 16);        \
+        else if (mt == 1) MVLLM_F32(D, 1, N, I, 8);               \
+        else if (mt == 2) MVLLM_F32(D, 2, N, I, 8);               \
+        else MVLLM_F32(D, 4, N, I, 8);                            \
+    } while (0)
+    if (dual && nt == 2)
+        MVLLM_F32_MT(true, 2, kRowsF32);
+    else if (dual)
+        MVLLM_F32_MT(true, 1, kRowsF32);
+    else if (!i8 && nt == 2)
+        MVLLM_F32_MT(false, 2, kRowsF32);
+    else if (!i8)
+        MVLLM_F32_MT(false, 1, kRowsF32);
+    else if (wide8 && nt == 2)
+        MVLLM_F32_MT(false, 2, kRowsI8x16);
+    else if (wide8)
+        MVLLM_F32_MT(false, 1, kRowsI8x16);
+    else if (nt == 2)
+        MVLLM_F32_MT(false, 2, kRowsI8x4);
+    else
+        MVLLM_F32_MT(false, 1, kRowsI8x4);
+#undef MVLLM_F32_MT
 #undef MVLLM_F32
-#undef MVLLM_I8
     return hipGetLastError();
 }
 

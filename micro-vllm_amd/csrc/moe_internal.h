@@ -227,11 +227,13 @@ hipError_t launch_prep_planes(int fmt, int terms, const float *x, const int *row
 // 16-byte aligned weight and input rows.
 bool f32mm_fits(bool dual, int K, int O);
 // i8 (single only): w[mi] holds int8 rows [O][K] and s[mi] their f32 row scales (QuantMat
-// fmt 8); 4-byte aligned rows.
+// fmt 8); 4-byte aligned rows.  out2 (f32 rows, single only): K is split over two workgroups,
+// out and out2 get the sums of its first and second half.
 hipError_t launch_f32mm(bool dual, int mt, const ExpertWork *ew, const void *items, int n_items,
                         const ExpertWork *ew1, int nrows_all, const float *in,
                         const int *in_rows, float *out, int mi, int K, int O, int act,
-                        float act_a, float act_b, hipStream_t st, bool i8 = false);
+                        float act_a, float act_b, hipStream_t st, bool i8 = false,
+                        float *out2 = nullptr);
 // Router tail: scores -> sigmoid in place (the mix), choice = mix + bias; then w *= rscale.
 hipError_t launch_route_tail(float *scores, const float *bias, float *choice, int n, int E,
                              hipStream_t st);

@@ -61,6 +61,9 @@ F32_CASES = [
     (7168, 2048, [1], 1, 2, 4.0, 25.0),             # K3 shared expert (SiTU), one token
     (6144, 2048, [3], 3, 1, 7.0, 0.0),              # GLM shared expert shape
     (1024, 512, [40, 5, 70], 80, 0, 0.0, 0.0),      # prefill rows: 16-, 32- and 64-row items
+    (32, 16, [1], 1, 0, 0.0, 0.0),                  # one K block, one tile
+    (4128, 272, [17, 16], 40, 1, 7.0, 0.0),         # K of unequal wave ranges, 8-column tiles
+    (4160, 3600, [2], 2, 2, 4.0, 25.0),             # 16-column dual tiles, 16 waves
 ]
 
 
@@ -122,7 +125,9 @@ def test_router_matches_host_router(hip, orc, T, D, E, k, rscale, bias):
                                        (4, 2048, 6144, 1), (4, 512, 1024, 40),
                                        (7, 7168, 2048, 3), (7, 256, 512, 70),
                                        (8, 2048, 7168, 1), (8, 7168, 2048, 4),
-                                       (8, 7168, 7168, 1), (8, 96, 48, 37)])
+                                       (8, 7168, 7168, 1), (8, 96, 48, 37),
+                                       (0, 32, 16, 1), (0, 480, 1040, 17), (0, 7200, 4112, 16),
+                                       (8, 160, 4160, 33), (8, 7200, 4096, 2), (8, 32, 80, 65)])
 def test_linear(hip, orc, fmt, O, K, n):
     """fmt 8 (QuantMat's int8 rows, MVLLM_DENSE_BITS=8) at K3's latent shapes, with codes
     and scales from the reference's quantizer rule (row amax / 127, clamp +-127) and an
@@ -245,3 +250,18 @@ def test_k3_latent_chain(hip, orc):
     err = npref.rel_err(got, uph_o)
     say("  rel_err", err)
     assert err < 1e-4
+
+
+def test_linear_int8_rows_aligned_to_four_bytes(hip, orc):
+    """int8 rows whose base is only 4-byte aligned take 4 codes a load instead of 16."""
+    rng = np.random.default_rng(88)
+    O, K, n = 64, 256, 5
+    x = rng.standard_normal((n, K)).astype(np.float32)
+    w = rng.integers(-127, 128, (O, K)).astype(np.int8)
+    sc = rng.uniform(0.001, 0.01, O).astype(np.float32)
+    raw = torch.zeros(O * K + 16, dtype=torch.int8, device="cuda")
+    raw[4:4 + O * K] = dev(w).reshape(-1)
+    y = torch.zeros((n, O), dtype=torch.float32, device="cuda")
+    hip.linear_dev(8, raw.data_ptr() + 4, dev(sc), O, K, dev(x), n, y)
+    torch.cuda.synchronize()
+    assert npref.rel_err(y.cpu().numpy(), orc.matmul(8, x, w, sc)) < TOL_F32
