@@ -6,7 +6,8 @@
 //
 //   k_moe_topk      one wave per token: k rounds of a wave-wide argmax under the
 //                   reference's order (larger score first, lower index on ties), then the
-//                   weights summed in pick order by every lane alike;
+//                   weights summed in pick order by every lane alike; for the router also
+//                   the sigmoid, the bias and the weights' scale;
 //   k_seg_count     per (token, slot): the expert's count of tokens whose summed weight
 //                   is non-zero, and its presence (union membership: any slot);
 //   k_seg_scan      one workgroup: experts in ascending id -> positions, row offsets,
@@ -14,7 +15,7 @@
 //   k_seg_rows      one workgroup per kept expert: its tokens in ascending order by a
 //                   ballot per 256 tokens (two chunks a pass), written at the expert's
 //                   row offset.
-#include "moe_internal.h"
+#include "mfma_common.h"
 
 #include <algorithm>
 
@@ -28,37 +29,116 @@ __device__ __forceinline__ bool rank_before(float va, int a, float vb, int b) {
 
 constexpr int kTopkWaves = 4;
 
-// NV > 0: the lane's scores (elements lane + 64 s, s < NV) stay in registers for all k
-// rounds (n_exp <= 64 NV); NV = 0 reads them again each round (up to 4096 experts).
-template <int NV>
+// A score as an unsigned key of the same order (-0 and +0 alike); 0 is kept for "taken".
+__device__ __forceinline__ uint32_t rank_key(float v) {
+    const uint32_t b = __float_as_uint(v + 0.f);  // -0 + 0 = +0
+    return max(b ^ ((uint32_t)((int)b >> 31) | 0x80000000u), 1u);
+}
+
+// Wave-wide maximum of non-negative keys, by row shifts and broadcasts (lane 63 ends with
+// it); a masked or missing source counts as 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t v) {
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+    v = dpp_max<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: lane 15 of each row
+    v = dpp_max<0x112, 0xf>(v);
+    v = dpp_max<0x114, 0xf>(v);
+    v = dpp_max<0x118, 0xf>(v);
+    v = dpp_max<0x142, 0xa>(v);  // row_bcast 15, 31
+    v = dpp_max<0x143, 0xc>(v);
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// NV > 0: the lane's scores (elements lane + 64 s, s < NV) stay in registers as keys for
+// all k rounds (n_exp <= 64 NV), each round one DPP maximum and a ballot: the chain of k
+// rounds is the whole time, and an argmax by twelve cross-lane LDS permutes a round took
+// 10 us at 384 experts, k = 8 (this one: 4.6, about a launch's own time).  NV = 0
+// reads the scores again each round (up to 4096 experts).
+// ROUTE: the router's tail in the same launch: choice (and part2, when K was split over two
+// workgroups) hold the router GEMM's sums, mix = sigmoid(sum) is written to mix_out, mix +
+// bias to choice_out, and the weights are scaled by rscale at the end
+// (src/gpu/metal_ops.cpp:218-231).  The sums may lie in mix_out and choice_out: a wave
+// reads its token's row before it writes it, and no other wave touches that row.
+template <int NV, bool ROUTE>
 __global__ __launch_bounds__(64 * kTopkWaves) void k_moe_topk(const float *choice,
                                                                 const float *mix, int n_tok,
                                                                 int n_exp, int k, int *idx,
-                                                                float *wt) {
+                                                                float *wt, const float *part2,
+                                                                const float *bias, float rscale,
+                                                                float *mix_out,
+                                                                float *choice_out) {
+    static_assert(!ROUTE || NV > 0, "the router's tail keeps its row in registers");
     const int tok = blockIdx.x * kTopkWaves + (int)(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (tok >= n_tok)  // wave-uniform
         return;
     const float *row = choice + (size_t)tok * n_exp;
-    float cv[NV > 0 ? NV : 1];
+    int mine = -1;  // lane i < k: the i-th pick
+    float w = 0.f;  // and its weight
+    if constexpr (NV > 0) {
+        uint32_t key[NV];
+        float mx[ROUTE ? NV : 1];
+        if constexpr (ROUTE) {
+            float sc[NV], s2[NV], bv[NV];
 #pragma unroll
-    for (int s = 0; s < NV; ++s)
-        cv[s] = lane + 64 * s < n_exp ? row[lane + 64 * s] : 0.f;
-    uint64_t taken = 0;  // bit s: element lane + 64 s is picked (n_exp <= 4096)
-    int mine = -1;       // lane i < k: the i-th pick
-    for (int i = 0; i < k; ++i) {
-        float bv = 0.f;
-        int bi = -1;
-        if constexpr (NV > 0) {
+            for (int s = 0; s < NV; ++s) {
+                const int j = min(lane + 64 * s, n_exp - 1);
+                sc[s] = row[j];
+                s2[s] = part2 ? part2[(size_t)tok * n_exp + j] : 0.f;
+                bv[s] = bias ? bias[j] : 0.f;
+            }
 #pragma unroll
             for (int s = 0; s < NV; ++s) {
                 const int j = lane + 64 * s;
-                if (j < n_exp && !((taken >> s) & 1u) && (bi < 0 || rank_before(cv[s], j, bv, bi))) {
-                    bv = cv[s];
-                    bi = j;
+                mx[s] = mf_sigmoid(part2 ? sc[s] + s2[s] : sc[s]);
+                const float c = mx[s] + bv[s];
+                key[s] = j < n_exp ? rank_key(c) : 0u;
+                if (j < n_exp) {
+                    mix_out[(size_t)tok * n_exp + j] = mx[s];
+                    choice_out[(size_t)tok * n_exp + j] = c;
                 }
             }
         } else {
+#pragma unroll
+            for (int s = 0; s < NV; ++s)
+                key[s] = lane + 64 * s < n_exp ? rank_key(row[lane + 64 * s]) : 0u;
+        }
+        for (int i = 0; i < k; ++i) {
+            uint32_t bk = 0;
+            int bs = 0;
+            float bm = 0.f;
+#pragma unroll
+            for (int s = 0; s < NV; ++s)
+                if (key[s] > bk) {  // the lane's lowest index on ties
+                    bk = key[s];
+                    bs = s;
+                    if constexpr (ROUTE)
+                        bm = mx[s];
+                }
+            const uint32_t m = wave_max(bk);
+            const uint64_t cand = __ballot(bk == m);
+            int win = __builtin_ctzll(cand);
+            if (cand & (cand - 1))  // equal scores in several lanes: the lowest index
+                win = (int)(~wave_max(bk == m ? ~(uint32_t)(bs * 64 + lane) : 0u) & 63u);
+            const int ws = __builtin_amdgcn_readlane(bs, win);
+            if (lane == win) {
+#pragma unroll
+                for (int s = 0; s < NV; ++s)
+                    key[s] = s == bs ? 0u : key[s];
+            }
+            const int wm = __builtin_amdgcn_readlane((int)__float_as_uint(bm), win);
+            if (lane == i) {
+                mine = ws * 64 + win;
+                w = __uint_as_float((uint32_t)wm);
+            }
+        }
+    } else {
+        uint64_t taken = 0;  // bit s: element lane + 64 s is picked (n_exp <= 4096)
+        for (int i = 0; i < k; ++i) {
+            float bv = 0.f;
+            int bi = -1;
             for (int s = 0; lane + 64 * s < n_exp; ++s) {
                 const int j = lane + 64 * s;
                 if ((taken >> s) & 1u)
@@ -69,35 +149,38 @@ __global__ __launch_bounds__(64 * kTopkWaves) void k_moe_topk(const float *choic
                     bi = j;
                 }
             }
-        }
-        // the order is total on the candidates, so any reduction tree finds the same one
+            // the order is total on the candidates, so any reduction tree finds the same one
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ov = __shfl_xor(bv, off);
-            const int oi = __shfl_xor(bi, off);
-            if (oi >= 0 && (bi < 0 || rank_before(ov, oi, bv, bi))) {
-                bv = ov;
-                bi = oi;
+            for (int off = 32; off > 0; off >>= 1) {
+                const float ov = __shfl_xor(bv, off);
+                const int oi = __shfl_xor(bi, off);
+                if (oi >= 0 && (bi < 0 || rank_before(ov, oi, bv, bi))) {
+                    bv = ov;
+                    bi = oi;
+                }
             }
+            if ((bi & 63) == lane)
+                taken |= 1ull << (bi >> 6);
+            if (lane == i)
+                mine = bi;
         }
-        if ((bi & 63) == lane)
-            taken |= 1ull << (bi >> 6);
-        if (lane == i)
-            mine = bi;
     }
     // weights: clipped at 0, summed in pick order (every lane adds the same sequence)
-    float w = 0.f;
     if (lane < k) {
-        w = mix ? mix[(size_t)tok * n_exp + mine] : row[mine];
+        if constexpr (!ROUTE)
+            w = mix ? mix[(size_t)tok * n_exp + mine] : row[mine];
         if (w < 0.f)
             w = 0.f;
     }
     float sum = 0.f;
     for (int i = 0; i < k; ++i)
-        sum += __shfl(w, i);
+        sum += __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(w), i));
     if (lane < k) {
         idx[(size_t)tok * k + lane] = mine;
-        wt[(size_t)tok * k + lane] = sum > 0.f ? w / sum : 1.f / (float)k;
+        float v = sum > 0.f ? w / sum : 1.f / (float)k;
+        if constexpr (ROUTE)
+            v = rscale != 1.f ? v * rscale : v;
+        wt[(size_t)tok * k + lane] = v;
     }
 }
 
@@ -277,20 +360,44 @@ __global__ __launch_bounds__(256) void k_seg_rows(const int *idx, const float *w
     }
 }
 
+// NV of a row of n_exp scores: the smallest instance that holds it (0: none).
+#define MVLLM_TOPK(ROUTE, ...)                                                              \
+    do {                                                                                    \
+        const dim3 grid((unsigned)((n_tok + kTopkWaves - 1) / kTopkWaves));                 \
+        const dim3 block(64 * kTopkWaves);                                                  \
+        const int nv = (n_exp + 63) / 64;                                                   \
+        if (nv <= 1)                                                                        \
+            hipLaunchKernelGGL((k_moe_topk<1, ROUTE>), grid, block, 0, st, __VA_ARGS__);    \
+        else if (nv <= 2)                                                                   \
+            hipLaunchKernelGGL((k_moe_topk<2, ROUTE>), grid, block, 0, st, __VA_ARGS__);    \
+        else if (nv <= 4)                                                                   \
+            hipLaunchKernelGGL((k_moe_topk<4, ROUTE>), grid, block, 0, st, __VA_ARGS__);    \
+        else if (nv <= 6)                                                                   \
+            hipLaunchKernelGGL((k_moe_topk<6, ROUTE>), grid, block, 0, st, __VA_ARGS__);    \
+        else if (nv <= 8)                                                                   \
+            hipLaunchKernelGGL((k_moe_topk<8, ROUTE>), grid, block, 0, st, __VA_ARGS__);    \
+        else                                                                                \
+            hipLaunchKernelGGL((k_moe_topk<0, false>), grid, block, 0, st, __VA_ARGS__);    \
+    } while (0)
+
 hipError_t launch_moe_topk(const float *choice, const float *mix, int n_tok, int n_exp, int k,
                            int *idx, float *wt, hipStream_t st) {
     if (n_tok < 1 || n_exp < 1 || n_exp > kRouteMaxExperts || k < 1 || k > 64 || k > n_exp)
         return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((n_tok + kTopkWaves - 1) / kTopkWaves)), block(64 * kTopkWaves);
-    const int nv = (n_exp + 63) / 64;
-    if (nv <= 2)
-        hipLaunchKernelGGL(k_moe_topk<2>, grid, block, 0, st, choice, mix, n_tok, n_exp, k, idx, wt);
-    else if (nv <= 8)
-        hipLaunchKernelGGL(k_moe_topk<8>, grid, block, 0, st, choice, mix, n_tok, n_exp, k, idx, wt);
-    else
-        hipLaunchKernelGGL(k_moe_topk<0>, grid, block, 0, st, choice, mix, n_tok, n_exp, k, idx, wt);
+    MVLLM_TOPK(false, choice, mix, n_tok, n_exp, k, idx, wt, nullptr, nullptr, 1.f, nullptr,
+               nullptr);
     return hipGetLastError();
 }
+
+hipError_t launch_route_topk(const float *sums, const float *sums2, const float *bias,
+                             float rscale, int n_tok, int n_exp, int k, float *mix,
+                             float *choice, int *idx, float *wt, hipStream_t st) {
+    if (n_tok < 1 || n_exp < 1 || n_exp > kRouteTopkMax || k < 1 || k > 64 || k > n_exp)
+        return hipErrorInvalidValue;
+    MVLLM_TOPK(true, sums, nullptr, n_tok, n_exp, k, idx, wt, sums2, bias, rscale, mix, choice);
+    return hipGetLastError();
+}
+#undef MVLLM_TOPK
 
 hipError_t launch_moe_segments(const int *idx, const float *wt, int n_tok, int topk, int n_exp,
                                int *work, int *eids, int *xoff, int *nr, int *rows, float *rw,

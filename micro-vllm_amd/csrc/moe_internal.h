@@ -80,6 +80,13 @@ hipError_t launch_quantize_mxfp4(const float *x, int n, int K, uint8_t *codes, u
 constexpr int kRouteMaxExperts = 4096;
 hipError_t launch_moe_topk(const float *choice, const float *mix, int n_tok, int n_exp, int k,
                            int *idx, float *wt, hipStream_t st);
+// The router's tail and top-k in one launch (n_exp <= kRouteTopkMax): sums (and sums2, added
+// to them, when not null) are the router GEMM's scores; mix = sigmoid, choice = mix + bias,
+// the top k of choice with weights from mix times rscale.  sums may be mix, sums2 choice.
+constexpr int kRouteTopkMax = 512;
+hipError_t launch_route_topk(const float *sums, const float *sums2, const float *bias,
+                             float rscale, int n_tok, int n_exp, int k, float *mix,
+                             float *choice, int *idx, float *wt, hipStream_t st);
 hipError_t launch_moe_segments(const int *idx, const float *wt, int n_tok, int topk, int n_exp,
                                int *work, int *eids, int *xoff, int *nr, int *rows, float *rw,
                                int cap_experts, int cap_rows, int *counts, hipStream_t st);

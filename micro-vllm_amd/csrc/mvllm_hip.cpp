@@ -2440,9 +2440,28 @@ int mvllm_hip_router_dev(const float *x, const float *w, const float *bias, int 
     hipStream_t st = static_cast<hipStream_t>(stream);
     ExpertWork ew{};
     ew.w[0] = w;
-    const int mt = n_tok <= 16 ? 1 : n_tok <= 32 ? 2 : 4;
+    // Up to kRouteTopkMax experts the sigmoid, the bias, the scale and the top-k are one launch
+    // (1 token, 384 experts of 7168: 35 -> 27 us).  A long K is then split over two workgroups,
+    // whose sums meet there, in the caller's two workspaces (27 -> 18 us; below D = 2048 the
+    // halves are too short to gain).  Few experts make few column tiles, so the row blocks
+    // are the smallest that keep the launch within one workgroup a CU: 61 tokens of the same
+    // router 23 us in blocks of 16 rows, 29 of 32, 42 of 64; 100 tokens 37 / 29 / 44 us,
+    // 200 tokens 52 / 51 / 44 us.
+    const bool fused = n_exp <= kRouteTopkMax, split = fused && D >= 2048;
+    int mt = 1;
+    auto tasks = [&] {
+        return (long long)((n_tok + 16 * mt - 1) / (16 * mt)) * (n_exp / 16) << (split ? 1 : 0);
+    };
+    while (mt < 4 && tasks() > 256)
+        mt *= 2;
+    float *half2 = split && tasks() <= 256 ? choice : nullptr;
     HIP_TRY(launch_f32mm(false, mt, nullptr, nullptr, 0, &ew, n_tok, x, nullptr, scores, 0, D,
-                         n_exp, 0, 0.f, 0.f, st));
+                         n_exp, 0, 0.f, 0.f, st, false, half2));
+    if (fused) {
+        HIP_TRY(launch_route_topk(scores, half2, bias, rscale, n_tok, n_exp, k, scores, choice,
+                                  idx, wt, st));
+        return 1;
+    }
     HIP_TRY(launch_route_tail(scores, bias, choice, n_tok, n_exp, st));
     HIP_TRY(launch_moe_topk(choice, scores, n_tok, n_exp, k, idx, wt, st));
     if (rscale != 1.f)

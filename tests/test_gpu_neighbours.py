@@ -85,7 +85,12 @@ def test_fmt0_block_on_f32_matrix_cores(hip, orc, case):
 
 @pytest.mark.parametrize("T,D,E,k,rscale,bias", [(1, 7168, 384, 8, 2.5, True),
                                                  (16, 2048, 64, 8, 1.0, False),
-                                                 (300, 1024, 256, 8, 1.0, True)])
+                                                 (300, 1024, 256, 8, 1.0, True),
+                                                 (61, 2064, 384, 8, 2.5, True),
+                                                 (100, 2048, 320, 64, 2.5, False),
+                                                 (33, 2048, 512, 3, 1.0, True),
+                                                 (5, 2048, 544, 4, 2.5, True),
+                                                 (1, 48, 32, 31, 2.5, True)])
 def test_router_matches_host_router(hip, orc, T, D, E, k, rscale, bias):
     say("router", T, D, E, k)
     rng = np.random.default_rng(T + D + E)
