@@ -178,7 +178,8 @@ def test_linear_refuses_odd_shapes(hip):
     assert b"linear_dev" in hip.lib().mvllm_hip_last_error()
 
 
-@pytest.mark.parametrize("rows,n,with_w", [(1, 7168, True), (9, 2048, True), (4, 333, False)])
+@pytest.mark.parametrize("rows,n,with_w", [(1, 7168, True), (9, 2048, True), (4, 333, False),
+                                           (2, 4, True), (3, 2052, False), (2, 8192, True)])
 def test_rmsnorm(hip, orc, rows, n, with_w):
     say("rmsnorm", rows, n)
     rng = np.random.default_rng(rows + n)
@@ -190,6 +191,27 @@ def test_rmsnorm(hip, orc, rows, n, with_w):
     err = npref.rel_err(y.cpu().numpy(), orc.rmsnorm(x, w, 1e-6))
     say("  rel_err", err)
     assert err < 2e-6
+
+
+@pytest.mark.parametrize("n,off", [(8196, 0), (16384, 0), (16388, 0), (2048, 1)])
+def test_rmsnorm_against_64_bits(hip, n, off):
+    """The last row in registers, the first in the loop, and rows that are not 16-byte
+    aligned, against 64 bits (the host's sequential f32 sum is itself 2.5e-6 off at 16384).
+    The register form's sum has at most 16 + 6 + 16 roundings of positive terms, the loop's
+    ceil(n / 256) + 6 + 4, each 2^-24; the norm takes half of that, and four more roundings
+    follow: below 2.9e-6."""
+    rng = np.random.default_rng(n + off)
+    x = (rng.standard_normal((2, n)) * 3).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    raw = torch.empty(2 * n + 1, device="cuda")
+    xd = raw[off:off + 2 * n].view(2, n)
+    xd.copy_(dev(x))
+    y = torch.zeros((2, n), dtype=torch.float32, device="cuda")
+    hip.rmsnorm_dev(xd, dev(w), y, 2, n, 1e-6)
+    torch.cuda.synchronize()
+    x64 = x.astype(np.float64)
+    exp = x64 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + 1e-6) * w
+    assert npref.rel_err(y.cpu().numpy(), exp) < 2.9e-6
 
 
 def test_k3_latent_chain(hip, orc):
