@@ -130,7 +130,13 @@ def test_route_then_segments(hip, orc):
     check_segments(orc, gi, gw, got, E)
 
 
-@pytest.mark.parametrize("T,topk,E", [(50, 6, 20), (1, 8, 64), (700, 3, 1500)])
+@pytest.mark.parametrize("T,topk,E", [(50, 6, 20), (1, 8, 64), (700, 3, 1500),
+                                      # the one-workgroup form's edges: one pair, a whole
+                                      # wave of one expert, 1024 / 1025
+                                      # pairs, 1024 / 1025 experts
+                                      (1, 1, 1), (64, 1, 1), (100, 8, 3), (128, 8, 384),
+                                      (1025, 1, 7), (128, 8, 1024), (341, 3, 384),
+                                      (128, 8, 1025)])
 def test_segments_arbitrary_ids(hip, orc, T, topk, E):
     """ids with -1 entries, an expert twice in one token, zero and cancelling weights."""
     rng = np.random.default_rng(T * 7 + E)
