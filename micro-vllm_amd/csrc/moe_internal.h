@@ -249,6 +249,16 @@ hipError_t launch_scale(float *w, size_t count, float rscale, hipStream_t st);
 hipError_t launch_rmsnorm(const float *x, const float *w, float *y, int rows, int n, float eps,
                           hipStream_t st);
 
+// int4 / MXFP4 matrices of any width with exact f32 activations (kern_qrows.hip): items,
+// ew1, in_rows, mi and the outputs as launch_f32mm's (dual H and single Y are f32 rows).
+// Requires K % 16 == 0 (q_rows_fits), 16-byte aligned input rows, 8-byte aligned weights
+// and 4-byte aligned int4 scales; any O.
+bool q_rows_fits(int fmt, int K);
+hipError_t launch_q_rows(int fmt, bool dual, int mt, const ExpertWork *ew, const void *items,
+                         int n_items, const ExpertWork *ew1, int nrows_all, const float *in,
+                         const int *in_rows, float *out, int mi, int K, int O, int act,
+                         float act_a, float act_b, hipStream_t st);
+
 // Native MXFP4 GEMM (kern_fp4.hip): v_mfma_scale_f32_16x16x128_f8f6f4 with e2m1 activations
 // (codes [rcap][K/2] + ue8m0 scales [rcap][K/32], from launch_quantize_mxfp4) against the
 // MXFP4 weights as stored.  Items and workgroup tiling as launch_gemm (mt 4, 8 and 16; an

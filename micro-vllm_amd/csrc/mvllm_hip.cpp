@@ -198,6 +198,7 @@ struct CallCfg {
     bool gemm = false;        // grouped GEMM (prefill-shaped)
     bool fp4 = false;         // grouped GEMM on native MXFP4 activations (option fp4act)
     bool f32 = false;         // fmt 0: the f32 matrix-core GEMM (kern_f32.hip)
+    bool qrows = false;       // fmt 4 / 7 of other widths: exact f32 activations (kern_qrows.hip)
     bool atomic_combine = false;  // decode kernels: combine folded into down (float atomics)
     bool w16 = false;         // every weight pointer 16-byte aligned (the wide-tile GEMM)
     int terms = 2;            // bf16 terms per activation (3: exact, 2: 2^-17, 1: bf16)
@@ -208,7 +209,7 @@ struct CallCfg {
     std::vector<int> per[kGemmClasses];  // plan_gemm's per-class scratch
     // the default configuration, keeping the vectors' storage
     void reset() {
-        mfma = gemm = fp4 = f32 = atomic_combine = w16 = false;
+        mfma = gemm = fp4 = f32 = qrows = atomic_combine = w16 = false;
         terms = 2;
         gu = dn = PhaseCfg();
         items.clear();
@@ -516,11 +517,11 @@ bool add_phase(const Ctx &C, CallCfg &cc, PhaseCfg &ph, const Plan &P, size_t sp
 // smallest class that holds it; classes ordered by mt, experts ascending within each.
 void plan_gemm(CallCfg &cc, const Plan &P, size_t split, int fmt) {
     cc.terms = cc.terms >= 2 ? 2 : 1;
-    const int max_mt = cc.f32 ? 4 : cc.fp4 ? kFp4MaxMt : gemm_max_mt(fmt, cc.terms);
+    const int max_mt = cc.f32 ? 4 : cc.qrows ? 2 : cc.fp4 ? kFp4MaxMt : gemm_max_mt(fmt, cc.terms);
     const int bm = 16 * max_mt;
     // bf16 one-term GEMM: an expert of 33-64 rows (a last block of that size) runs as two
     // 32-row items of the two-workgroups-per-CU class, which read its weights together
-    const bool split64 = !cc.f32 && !cc.fp4 && cc.terms == 1 && max_mt >= 4;
+    const bool split64 = !cc.f32 && !cc.qrows && !cc.fp4 && cc.terms == 1 && max_mt >= 4;
     std::vector<int> *per = cc.per;  // class index = log2(mt)
     for (int c = 0; c < kGemmClasses; ++c)
         per[c].clear();
@@ -574,7 +575,7 @@ void plan_gemm(CallCfg &cc, const Plan &P, size_t split, int fmt) {
         cc.items.insert(cc.items.end(), per[c].begin(), per[c].end());
         g.it1 = cc.items.size() / 4;
     }
-    cc.gemm = !cc.f32;
+    cc.gemm = !cc.f32 && !cc.qrows;
 }
 
 // ordered: the combine keeps the reference's expert order even for decode-shaped calls
@@ -640,6 +641,17 @@ void plan_call(const Ctx &C, CallCfg &cc, const Plan &P, int fmt, int D, int I, 
     }
     if (gok && C.gemm != 2) {  // decode-shaped call the decode kernels do not fit: keep
         cc.terms = C.mode == 2 ? 1 : 2;  // the decode accuracy (2 terms) unless mode 2
+        plan_gemm(cc, P, split, fmt);
+        return;
+    }
+    // other widths and alignments: the matrix cores on exact f32 activations; what is left
+    // (odd widths, rows of 4-byte alignment) takes the element-wise kernel
+    bool qok = q_rows_fits(fmt, D) && q_rows_fits(fmt, I) && aligned(in, 16);
+    for (const ExpertWork &w : P.ew)
+        for (int m = 0; m < 3; ++m)
+            qok = qok && aligned(w.w[m], 8) && (fmt != 4 || aligned(w.s[m], 4));
+    if (qok) {
+        cc.qrows = true;
         plan_gemm(cc, P, split, fmt);
     }
 }
@@ -1037,9 +1049,8 @@ int run_phases(Ctx &C, const Plan &P, const CallCfg &cc, const DevPlan &dp, cons
                                         st));
             C.stats[14] += 1;
         }
-    } else if (cc.f32) {
-        // f32 matrix cores on the f32 rows themselves (no planes): gate/up + act -> H f32,
-        // down -> Y
+    } else if (cc.f32 || cc.qrows) {
+        // matrix cores on the f32 rows themselves (no planes): gate/up + act -> H f32, down -> Y
         HIP_TRY(mark(1));
         for (int part = 0; part < 2; ++part) {
             if (part == 1 && gate_event)
@@ -1049,9 +1060,13 @@ int run_phases(Ctx &C, const Plan &P, const CallCfg &cc, const DevPlan &dp, cons
                 const size_t i0 = part ? g.it_split : g.it0, i1 = part ? g.it1 : g.it_split;
                 if (i1 <= i0)
                     continue;
-                HIP_TRY(launch_f32mm(true, g.mt, dp.ew, dp.items + 4 * i0,
-                                     static_cast<int>(i1 - i0), nullptr, 0, in, in_rows,
-                                     static_cast<float *>(B.H), 0, D, I, act, a, b, st));
+                const int ni = static_cast<int>(i1 - i0);
+                float *H = static_cast<float *>(B.H);
+                HIP_TRY(cc.qrows ? launch_q_rows(fmt, true, g.mt, dp.ew, dp.items + 4 * i0, ni,
+                                                 nullptr, 0, in, in_rows, H, 0, D, I, act, a, b,
+                                                 st)
+                                 : launch_f32mm(true, g.mt, dp.ew, dp.items + 4 * i0, ni, nullptr,
+                                                0, in, in_rows, H, 0, D, I, act, a, b, st));
                 C.stats[13] += 1;
             }
         }
@@ -1059,10 +1074,13 @@ int run_phases(Ctx &C, const Plan &P, const CallCfg &cc, const DevPlan &dp, cons
         HIP_TRY(mark(3));
         for (int c = 0; c < cc.n_gcls; ++c) {
             const GemmCls &g = cc.gcls[c];
-            HIP_TRY(launch_f32mm(false, g.mt, dp.ew, dp.items + 4 * g.it0,
-                                 static_cast<int>(g.it1 - g.it0), nullptr, 0,
-                                 static_cast<const float *>(B.H), nullptr,
-                                 static_cast<float *>(B.Y), 2, I, D, 0, 0.f, 0.f, st));
+            const int ni = static_cast<int>(g.it1 - g.it0);
+            const float *H = static_cast<const float *>(B.H);
+            float *Y = static_cast<float *>(B.Y);
+            HIP_TRY(cc.qrows ? launch_q_rows(fmt, false, g.mt, dp.ew, dp.items + 4 * g.it0, ni,
+                                             nullptr, 0, H, nullptr, Y, 2, I, D, 0, 0.f, 0.f, st)
+                             : launch_f32mm(false, g.mt, dp.ew, dp.items + 4 * g.it0, ni, nullptr,
+                                            0, H, nullptr, Y, 2, I, D, 0, 0.f, 0.f, st));
             C.stats[14] += 1;
         }
     } else if (cc.gemm) {

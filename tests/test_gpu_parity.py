@@ -202,6 +202,14 @@ DEV_CASES = [
     (0, 64, 48, [2, 1], 3, 1, 3.0, 0.0, (0,), 0),                  # f32 weights
     (4, 2048, 1024, [7, 1, 13], 16, 1, 7.0, 0.0, (), 0),           # rows > one item
     (7, 2048, 1024, [5, 9], 12, 2, 4.0, 25.0, (), 0),
+    # widths that are no multiples of 256: partial 64-blocks of K (16, 32, 48), O past a tile,
+    # 16- and 32-row items, an empty expert, skips
+    (4, 16, 48, [1], 1, 0, 0.0, 0.0, (), 0),
+    (7, 48, 16, [3], 3, 2, 4.0, 25.0, (), 0),
+    (4, 208, 176, [17, 16, 33], 40, 1, 7.0, 0.0, (), 2),
+    (7, 2080, 1056, [1, 0, 33, 16], 40, 2, 4.0, 25.0, (2,), 1),
+    (4, 2112, 704, [2] * 24, 12, 0, 0.0, 0.0, (), 0),              # four-tile waves
+    (7, 2112, 720, [1] * 24, 5, 2, 4.0, 25.0, (), 0),
 ]
 
 
@@ -310,11 +318,12 @@ def test_validation_matches_reference(hip):
     assert hip.moe_block(*args, 0, 0.0, 0.0) == 1 and np.array_equal(o, c.out)
 
 
-@pytest.mark.parametrize("D,I", [(256, 128), (512, 512)])
+@pytest.mark.parametrize("D,I", [(256, 128), (512, 512), (250, 130), (560, 304)])
 def test_nonfinite_propagation(hip, orc, D, I):
     """Inf scales / activations: NaN and Inf land where the reference puts them, on the
-    element-wise path (256 x 128) and through the matrix-core decode kernels (512 x 512:
-    chains over n - 8, exact redo of tiles with out-of-range scales)."""
+    element-wise path (250 x 130), through the matrix-core decode kernels (512 x 512:
+    chains over n - 8, exact redo of tiles with out-of-range scales) and through the
+    kernels of other widths (256 x 128; 560 x 304 with partial K blocks)."""
     say("nonfinite", D, I)
     rng = np.random.default_rng(8)
     for fmt in (4, 7):
@@ -337,14 +346,16 @@ def test_nonfinite_propagation(hip, orc, D, I):
 
 
 @pytest.mark.parametrize("fmt", [4, 7])
-@pytest.mark.parametrize("path,D,I,gemm", [("elementwise", 256, 128, 0), ("decode", 512, 512, 2),
+@pytest.mark.parametrize("path,D,I,gemm", [("elementwise", 250, 130, 0), ("widths", 256, 128, 0),
+                                           ("decode", 512, 512, 2),
                                            ("gemm", 512, 256, 1)])
 def test_clamp_swiglu_nonfinite_up(hip, orc, fmt, path, D, I, gemm):
     """ClampSwiGLU with a non-finite up projection: the reference clamps `up` with
     comparisons (src/quant/quant.hpp:37-50), so a NaN up stays NaN and reaches the row's
     down outputs; an infinite one is clamped to +-limit.  The up scales alone carry the
     non-finite values (MXFP4 byte 255 on a zero nibble gives 0 * inf = NaN; an int4 scale
-    of inf or NaN), on the element-wise, decode and grouped-GEMM paths."""
+    of inf or NaN), on the element-wise, decode and grouped-GEMM paths and the one for other
+    widths."""
     say("clamp nonfinite up", fmt, path)
     rng = np.random.default_rng(19 + fmt + D)
     c = random_case(rng, fmt, D, I, [2, 1, 3], 6, 1, 7.0, 0.0)

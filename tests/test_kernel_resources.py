@@ -59,6 +59,7 @@ def test_gemm_classes_within_register_budget(tmp_path):
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
 @pytest.mark.parametrize("src,kernel", [("kern_fp4.hip", "k_gemm_fp4"),
                                         ("kern_f32.hip", "k_f32mm"),
+                                        ("kern_qrows.hip", "k_q_rows"),
                                         ("kern_wide.hip", "k_gemm_wide<true, 8, 4, 8>"),
                                         ("kern_wide.hip", "k_gemm_wide<false, 8, 4, 8>")])
 def test_other_gemms_spill_free(tmp_path, src, kernel):
