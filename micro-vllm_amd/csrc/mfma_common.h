@@ -90,15 +90,20 @@ __device__ __forceinline__ bf16x8 decode_b7_exact(uint32_t w, float scale7) {
 
 // int4 nibbles n of one dword -> bf16(n - 8), in decode_b<4>'s slot order, exact: each
 // byte becomes the e4m3 code of (n - 8) * 2^-9 (sign bit and 8 - n for n < 8), which the
-// converter scales back by 2^9.
-__device__ __forceinline__ uint32_t int4_signed_codes(uint32_t l) {  // bytes 0..15
-    const uint32_t ge8 = ((l >> 3) & 0x01010101u) * 0xffu;
-    const uint32_t neg = 0x80808080u | ((~l & 0x07070707u) + 0x01010101u);
-    return (ge8 & (l & 0x07070707u)) | (~ge8 & neg);
+// converter scales back by 2^9.  Five instructions per four nibbles (the low ones of the
+// bytes of l; the high ones are ignored): the codes of n < 8 by a byte permute of their
+// table, a byte mask of n < 8 by another (selector 0: byte 0xff, selector 8: the sign of a
+// zero byte), and a bit select.  Shifts, adds and a multiply took ten, and the decode is what
+// the vector ALU does beside the matrix cores here.
+__device__ __forceinline__ uint32_t int4_signed_codes(uint32_t l) {
+    const uint32_t n7 = l & 0x07070707u;
+    const uint32_t neg = __builtin_amdgcn_perm(0x81828384u, 0x85868788u, n7);
+    const uint32_t lt8 = __builtin_amdgcn_perm(0u, 0xffu, l & 0x08080808u);
+    return (lt8 & neg) | (~lt8 & n7);
 }
 __device__ __forceinline__ bf16x8 decode_b4_signed(uint32_t w) {
-    const int lo = (int)int4_signed_codes(w & 0x0F0F0F0Fu);
-    const int hi = (int)int4_signed_codes((w >> 4) & 0x0F0F0F0Fu);
+    const int lo = (int)int4_signed_codes(w);
+    const int hi = (int)int4_signed_codes(w >> 4);
     return pack8(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.f, false),
                  __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.f, true),
                  __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.f, false),
