@@ -142,8 +142,7 @@ struct Resident {
     size_t bytes = 0;
     void *dev = nullptr;
     hipEvent_t ready = nullptr;    // copy finished (copy stream)
-    hipEvent_t last_use = nullptr; // last compute that read it
-    bool used = false;
+    bool landed = false;           // ready was seen complete: readers need no wait
     std::list<long long>::iterator lru;
 };
 
@@ -231,10 +230,10 @@ struct Ctx {
     hipEvent_t miss_done = nullptr;  // the staged path's miss copies (copy stream)
     void *scratch_ptr = nullptr;     // device address of `scratch` on `device`
     bool have_last = false;
-    DevBuf H, Y, Xc, Oc, miss, Ph, HP, Xp;
+    DevBuf H, Y, Xc, miss, Ph, HP, Xp;
     DevBuf Lp;  // planes of mvllm_hip_linear_dev's input rows
     DevBuf Rp;  // device plan of mvllm_hip_moe_block_routed_dev
-    HostBuf hx, ho;
+    HostBuf hx;
     // the plan and configuration of the current call (every entry holds mu), reused
     Plan plan;
     CallCfg cfg;
@@ -1295,10 +1294,10 @@ void res_drop(Ctx &C, long long key) {
     if (it == C.res.end())
         return;
     Resident &r = it->second;
-    // the block is recycled only after readers and the copy are done: the copy
-    // stream waits for the last reader before writing into a recycled block
-    if (r.used)
-        (void)hipStreamWaitEvent(C.copy, r.last_use, 0);
+    // The block is recycled only after readers and the copy are done.  Calls of
+    // mvllm_hip_moe_block have ended (each drains its stream before it returns, under the
+    // lock held here); the copy stream waits for the layer's table readers before it
+    // writes into a recycled block.
     auto lu = C.layer_use.find(r.layer);
     if (lu != C.layer_use.end())
         (void)hipStreamWaitEvent(C.copy, lu->second, 0);
@@ -1313,7 +1312,6 @@ void res_drop(Ctx &C, long long key) {
         C.by_host.erase(r.host);
     C.lru.erase(r.lru);
     (void)hipEventDestroy(r.ready);
-    (void)hipEventDestroy(r.last_use);
     C.res.erase(it);
     C.stats[8] += 1;
 }
@@ -1400,10 +1398,8 @@ void mvllm_hip_shutdown(void) {
     C.Lp.release();
     C.Rp.release();
     C.Xc.release();
-    C.Oc.release();
     C.miss.release();
     C.hx.release();
-    C.ho.release();
     for (auto &s : C.slots) {
         s.host.release();
         s.dev.release();
@@ -1564,21 +1560,34 @@ int mvllm_hip_moe_block(int nb, int D, int Iinter, int fmt, int qgs, const void 
     hipStream_t st = C.own;
     if (!order_after_previous(C, st))
         return 0;
+    // Whatever ends this call, its stream is idle when it returns: the resident blobs it
+    // reads may be dropped and their blocks rewritten by the next entry.
+    struct Drain {
+        hipStream_t st;
+        ~Drain() {
+            if (st)
+                (void)hipStreamSynchronize(st);
+        }
+    } drain{st};
 
     // 1) resolve expert pieces: resident blobs first, misses copied into the arena
     const size_t pb[4] = {piece_bytes(fmt, 0, D, Iinter), piece_bytes(fmt, 1, D, Iinter),
                           piece_bytes(fmt, 2, D, Iinter), piece_bytes(fmt, 3, D, Iinter)};
     std::vector<ExpertWork> hit, miss;
-    std::vector<std::vector<int>> hit_rows;  // unused; order kept by row0
-    std::vector<Resident *> touched;
     std::vector<std::pair<const void *, size_t>> miss_src;  // per miss expert: 6 pieces
     for (const ExpertWork &w0 : P.ew) {
         ExpertWork w = w0;
         bool all = true;
         Resident *rs[6] = {};
+        // an expert's pieces usually lie in one blob: look only for those outside the last
+        auto find = [&](const void *p, Resident *last) {
+            const uint8_t *b = static_cast<const uint8_t *>(p);
+            return last && b >= last->host && b < last->host + last->bytes ? last
+                                                                           : res_lookup(C, p);
+        };
         for (int m = 0; m < 3 && all; ++m) {
-            rs[2 * m] = res_lookup(C, w.w[m]);
-            rs[2 * m + 1] = fmt ? res_lookup(C, w.s[m]) : rs[2 * m];
+            rs[2 * m] = find(w.w[m], m ? rs[2 * m - 1] : nullptr);
+            rs[2 * m + 1] = fmt ? find(w.s[m], rs[2 * m]) : rs[2 * m];
             const size_t bw = pb[m == 2 ? 2 : 0], bs = pb[m == 2 ? 3 : 1];
             all = rs[2 * m] &&
                   static_cast<const uint8_t *>(w.w[m]) + bw <= rs[2 * m]->host + rs[2 * m]->bytes &&
@@ -1593,12 +1602,23 @@ int mvllm_hip_moe_block(int nb, int D, int Iinter, int fmt, int qgs, const void 
                     w.s[m] = static_cast<uint8_t *>(rs[2 * m + 1]->dev) +
                              (static_cast<const uint8_t *>(w.s[m]) - rs[2 * m + 1]->host);
             }
-            for (auto *r : rs)
-                if (r) {
-                    HIP_TRY(hipStreamWaitEvent(st, r->ready, 0));
-                    touched.push_back(r);
-                    C.lru.splice(C.lru.begin(), C.lru, r->lru);
+            // wait for a blob's copy once, and only while it has not been seen complete (a
+            // wait is a queue packet: six an expert and an event after the call for each
+            // took 0.7 ms of a call on 25 experts)
+            for (int k = 0; k < 6; ++k) {
+                Resident *r = rs[k];
+                if (k && r == rs[k - 1])
+                    continue;
+                if (!r->landed) {
+                    const hipError_t q = hipEventQuery(r->ready);
+                    r->landed = q == hipSuccess;
+                    if (q == hipErrorNotReady)
+                        HIP_TRY(hipStreamWaitEvent(st, r->ready, 0));
+                    else
+                        HIP_TRY(q);
                 }
+                C.lru.splice(C.lru.begin(), C.lru, r->lru);
+            }
             hit.push_back(w);
             C.stats[6] += 1;
         } else {
@@ -1677,50 +1697,41 @@ int mvllm_hip_moe_block(int nb, int D, int Iinter, int fmt, int qgs, const void 
     P.ew.insert(P.ew.end(), hit.begin(), hit.end());
     P.ew.insert(P.ew.end(), miss.begin(), miss.end());
 
-    // 3) activations: gather the compact rows into pinned memory, one H2D copy
-    const size_t R = P.xrow.size();
-    HIP_TRY(C.hx.ensure(R * D * 4));
-    HIP_TRY(C.Xc.ensure(R * D * 4));
+    // 3) the compact activation rows, then the destination rows of out (combine writes
+    // out_row = t), gathered into pinned memory: one H2D copy
+    const size_t R = P.xrow.size(), T = P.out_row.size();
+    const size_t xb = (R * D * 4 + 255) & ~size_t(255), ob = T * D * 4;
+    HIP_TRY(C.hx.ensure(xb + ob));
+    HIP_TRY(C.Xc.ensure(xb + ob));
+    float *hx = static_cast<float *>(C.hx.p), *ho = hx + xb / 4;
+    float *dx = static_cast<float *>(C.Xc.p), *dout = dx + xb / 4;
     for (size_t j = 0; j < R; ++j)
-        std::memcpy(static_cast<float *>(C.hx.p) + j * D, xg + (size_t)P.xrow[j] * D,
-                    (size_t)D * 4);
-    HIP_TRY(hipMemcpyAsync(C.Xc.p, C.hx.p, R * D * 4, hipMemcpyHostToDevice, st));
-    // 4) the destination rows of out, compacted (combine writes out_row = t)
-    const size_t T = P.out_row.size();
-    HIP_TRY(C.ho.ensure(T * D * 4));
-    HIP_TRY(C.Oc.ensure(T * D * 4));
+        std::memcpy(hx + j * D, xg + (size_t)P.xrow[j] * D, (size_t)D * 4);
     for (size_t t = 0; t < T; ++t)
-        std::memcpy(static_cast<float *>(C.ho.p) + t * D, out + (size_t)P.out_row[t] * D,
-                    (size_t)D * 4);
-    HIP_TRY(hipMemcpyAsync(C.Oc.p, C.ho.p, T * D * 4, hipMemcpyHostToDevice, st));
+        std::memcpy(ho + t * D, out + (size_t)P.out_row[t] * D, (size_t)D * 4);
+    HIP_TRY(hipMemcpyAsync(dx, hx, xb + ob, hipMemcpyHostToDevice, st));
     C.stats[3] += static_cast<double>((R + T) * D * 4);
     std::vector<int> dest_rows = P.out_row;
     for (size_t t = 0; t < T; ++t)
         P.out_row[t] = static_cast<int>(t);
     CallCfg &cc = C.cfg;
-    plan_call(C, cc, P, fmt, D, Iinter, hit.size(), C.Xc.p, true);
+    plan_call(C, cc, P, fmt, D, Iinter, hit.size(), dx, true);
     Bufs B;
     HIP_TRY(get_bufs(C, cc, R, D, Iinter, B));
     DevPlan dp{};
     if (!upload_plan(C, P, cc, st, dp, true))
         return 0;
-    const int ok = run_phases(C, P, cc, dp, B, fmt, D, Iinter, act, act_a, act_b,
-                              static_cast<const float *>(C.Xc.p), nullptr,
-                              static_cast<float *>(C.Oc.p), st, hit.size(), miss_ev);
-    if (!ok)
+    if (!run_phases(C, P, cc, dp, B, fmt, D, Iinter, act, act_a, act_b, dx, nullptr, dout, st,
+                    hit.size(), miss_ev))
         return 0;
-    for (Resident *r : touched) {
-        HIP_TRY(hipEventRecord(r->last_use, st));
-        r->used = true;
-    }
-    HIP_TRY(hipMemcpyAsync(C.ho.p, C.Oc.p, T * D * 4, hipMemcpyDeviceToHost, st));
-    C.stats[4] += static_cast<double>(T * D * 4);
+    HIP_TRY(hipMemcpyAsync(ho, dout, ob, hipMemcpyDeviceToHost, st));
+    C.stats[4] += static_cast<double>(ob);
     if (!finish_call(C, st, dp.slot))
         return 0;
+    drain.st = nullptr;
     HIP_TRY(hipStreamSynchronize(st));
     for (size_t t = 0; t < T; ++t)
-        std::memcpy(out + (size_t)dest_rows[t] * D, static_cast<float *>(C.ho.p) + t * D,
-                    (size_t)D * 4);
+        std::memcpy(out + (size_t)dest_rows[t] * D, ho + t * D, (size_t)D * 4);
     return 1;
 }
 
@@ -1811,7 +1822,6 @@ int promote_locked(Ctx &C, const void *host_blob, size_t bytes, int layer, int e
     r.bytes = bytes;
     r.dev = dev;
     HIP_TRY(hipEventCreateWithFlags(&r.ready, hipEventDisableTiming));
-    HIP_TRY(hipEventCreateWithFlags(&r.last_use, hipEventDisableTiming));
     HIP_TRY(hipMemcpyAsync(dev, host_blob, bytes, hipMemcpyHostToDevice, C.copy));
     C.copy_epoch += 1;
     HIP_TRY(hipEventRecord(r.ready, C.copy));
