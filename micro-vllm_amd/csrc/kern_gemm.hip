@@ -40,6 +40,7 @@ struct GemmArgs {
     const GemmItem *items;  // per item (UNI kernels: none; one expert ew1 over nrows_all rows)
     ExpertWork ew1;
     int nrows_all;
+    int ks;                 // UNI: K splits (split s writes its sums to out + s nrows_all O)
     const __bf16 *pin;  // A planes [TERMS][rcap][K] (int4: 8-blocks in slot order)
     __bf16 *pout;       // dual: H planes [TERMS][rcap][O]
     float *out;         // single: Y [rcap][O] f32; dual: H [rcap][O] f32 instead of planes
@@ -104,6 +105,8 @@ struct TaskD {
     __amdgpu_buffer_rsrc_t rw[2], rs[2];
     uint32_t vw[2], vs[2];
     int jbase, nrow, col0;
+    int k0, nk;  // UNI: first K step (the offsets above include it) and number of steps
+    int orow;    // UNI: output row of input row 0 (each K split has its own output rows)
 };
 
 // One workgroup per task.  UNI: one expert (A.ew1) over rows [0, A.nrows_all) in blocks of
@@ -154,6 +157,15 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
         TaskD<FMT> d;
         int item = task / A.nbn;
         int nb = task - item * A.nbn;
+        if constexpr (UNI) {
+            // the column blocks of one (row block, K range) run side by side: they read the
+            // same planes through their L2.  Ranges are whole pairs of K steps.
+            const int np = (nk + 1) / 2, split = item % A.ks;
+            item /= A.ks;
+            d.k0 = 2 * (np * split / A.ks);
+            d.nk = min(2 * (np * (split + 1) / A.ks), nk) - d.k0;
+            d.orow = split * A.nrows_all;
+        }
         if constexpr (!UNI && MT <= 2) {
             // An expert's run of nblk items owns tasks [g0 nbn, (g0 + nblk) nbn); they go
             // column block by column block, its row blocks adjacent, so that the row blocks
@@ -187,6 +199,10 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
             d.vw[m] = (uint32_t)(trow + (lane >> 2)) * rowb + 8u * (uint32_t)(lane & 3);
             d.vs[m] = (uint32_t)(trow + (lane >> 2)) * srow +
                       (kChunkS ? 16u : FMT == 4 ? 8u : 4u) * (uint32_t)(lane & 3);
+            if constexpr (UNI) {
+                d.vw[m] += (uint32_t)d.k0 * 128u;
+                d.vs[m] += (uint32_t)(d.k0 >> 1) * (FMT == 4 ? 32u : 16u);
+            }
         }
         return d;
     };
@@ -239,15 +255,20 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
         u32x4 v[ACH];  // native vectors: copies of HIP's uint4 struct go through scratch
     };
     auto load_a = [&] __attribute__((always_inline)) (AStage &ra, const TaskD<FMT> &d, int k) {
-        // unconditional loads (rows past nrow re-read the last row; their results are
-        // never stored) keep the loop body free of branches
+        // the item's rows of each plane are one buffer resource: rows past nrow lie beyond it
+        // and load as zeros (their results are never stored), so the loop body has no branches
+        // and the offsets of a term's chunks serve every term
 #pragma unroll
         for (int u = 0; u < ACH; ++u) {
             const int c = u * kGemmThreads + tid;
-            const int tm = c / (BM * 32), r = min((c >> 5) % BM, d.nrow - 1), cc = c & 31;
-            ra.v[u] = *reinterpret_cast<const u32x4 *>(
-                A.pin + ((size_t)tm * rcap + d.jbase + r) * (size_t)K + (size_t)k * kGemmBK +
-                8 * cc);
+            const int tm = u * kGemmThreads / (BM * 32), r = (c >> 5) % BM, cc = c & 31;
+            const __amdgpu_buffer_rsrc_t rs =
+                buf_rsrc(A.pin + ((size_t)tm * rcap + d.jbase) * (size_t)K,
+                         (uint32_t)d.nrow * (uint32_t)K * 2u);
+            ra.v[u] = __builtin_bit_cast(
+                u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                           rs, (uint32_t)r * (uint32_t)K * 2u + 16u * (uint32_t)cc,
+                           (uint32_t)((UNI ? d.k0 : 0) + k) * (uint32_t)(kGemmBK * 2), 0));
         }
     };
     auto store_a = [&] __attribute__((always_inline)) (const AStage &ra, int buf) {
@@ -610,8 +631,9 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
                     }
                 } else {
                     if (r < d.nrow) {
-                        A.out[(size_t)j * O + d.col0 + t] = acc[mt][0][i];
-                        A.out[(size_t)j * O + d.col0 + 16 + t] = acc[mt][1][i];
+                        const size_t row = (size_t)((UNI ? d.orow : 0) + j);
+                        A.out[row * O + d.col0 + t] = acc[mt][0][i];
+                        A.out[row * O + d.col0 + 16 + t] = acc[mt][1][i];
                     }
                 }
             }
@@ -629,6 +651,7 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
         return;
     const int task = A.xcd ? xcd_task(blockIdx.x, n_tasks) : (int)blockIdx.x;
     const TaskD<FMT> cur = make_task(task);
+    const int ns = __builtin_amdgcn_readfirstlane(UNI ? cur.nk : nk);  // K steps of this task
     GStep<FMT> b0, b1;
     Scl sc, sn;  // scales of this pair of steps (chunk) / of the next pair (chunk)
     AStage ra0, ra1;
@@ -644,8 +667,8 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
         load_s(sn, cur, 0);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (PA == 2)
-            load_a(ra1, cur, min(1, nk - 1));
-        load_b(b1, cur, min(1, nk - 1));
+            load_a(ra1, cur, min(1, ns - 1));
+        load_b(b1, cur, min(1, ns - 1));
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (!kDmaA)
             store_a(ra0, 0);
@@ -656,7 +679,7 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
     // wrapping to the first steps instead re-read two steps of weights from HBM per task,
     // a quarter of the bytes at K = 2048.
     auto step_even = [&] __attribute__((always_inline)) (int k, auto exact) {
-        const int k2 = min(k + 2, nk - 1);
+        const int k2 = min(k + 2, ns - 1);
         if constexpr (kChunkS) {
             // a new chunk opens at this pair: the chunk loaded two steps ago
             if (((k >> 1) % PPC) == 0)
@@ -665,11 +688,11 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
             sc = sn;
         }
         if constexpr (kDmaA)
-            dma_a(cur, min(k + 1, nk - 1), 1);  // first: the barrier below waits for it only
+            dma_a(cur, min(k + 1, ns - 1), 1);  // first: the barrier below waits for it only
         else if constexpr (PA == 2)
             load_a(ra0, cur, k2);
         else
-            load_a(ra1, cur, min(k + 1, nk - 1));
+            load_a(ra1, cur, min(k + 1, ns - 1));
         compute(b0, 0, sc, k >> 1, 0, exact);
         __builtin_amdgcn_sched_barrier(0);
         load_b(b0, cur, k2);
@@ -680,13 +703,13 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
     };
     // odd step k + 1: LDS buffer 1, weights b1; stages A(k + 2) into buffer 0
     auto step_odd = [&] __attribute__((always_inline)) (int k, auto exact) {
-        const int k3 = min(k + 3, nk - 1);
+        const int k3 = min(k + 3, ns - 1);
         if constexpr (kDmaA)
-            dma_a(cur, min(k + 2, nk - 1), 0);
+            dma_a(cur, min(k + 2, ns - 1), 0);
         else if constexpr (PA == 2)
             load_a(ra1, cur, k3);
         else
-            load_a(ra0, cur, min(k + 2, nk - 1));
+            load_a(ra0, cur, min(k + 2, ns - 1));
         compute(b1, 1, sc, k >> 1, 1, exact);
         __builtin_amdgcn_sched_barrier(0);
         load_b(b1, cur, k3);
@@ -699,12 +722,12 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
     // loop head, on which the wait counts would also wait for step k + 1's weights.  An
     // odd last step runs after the loop.
     auto k_loop = [&] __attribute__((always_inline)) (auto exact) {
-        for (int k = 0; k + 2 <= nk; k += 2) {
+        for (int k = 0; k + 2 <= ns; k += 2) {
             step_even(k, exact);
             step_odd(k, exact);
         }
-        if (nk & 1)
-            step_even(nk - 1, exact);
+        if (ns & 1)
+            step_even(ns - 1, exact);
     };
     prologue();
     k_loop(std::false_type{});
@@ -863,8 +886,45 @@ hipError_t launch_gemm(int fmt, bool dual, int terms, int mt, const ExpertWork *
     return hipErrorInvalidValue;
 }
 
+// y[i] = sum over s < ks of part[s n + i], in order of s; n float4 (y: any float alignment)
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+__global__ __launch_bounds__(256) void k_sum_splits(const f4v *part, f4u *y, size_t n, int ks) {
+    const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
+    if (i >= n)
+        return;
+    f4v v = part[i];
+    for (int s = 1; s < ks; ++s)
+        v += part[(size_t)s * n + i];
+    y[i] = v;
+}
+
+// K splits of a dense linear.  Without them a launch had n / (16 mt) x O / 256 workgroups
+// (int4 2048 x 6144 at 512 rows: 64 on 256 CUs; 7168 x 7168 at 61 rows: 28).  The split of
+// least estimated time: rounds of workgroups (one per CU with 64 rows, whose planes fill the
+// LDS, two below) times a workgroup's pairs of K steps (measured 3.6, 5 and 8 us each with 16,
+// 32 and 64 rows), plus the launch that adds the sums and their bytes.  Per call with its
+// planes, unsplit -> split: int4 2048 x 6144 at 1 row 51 -> 15 us, at 100 rows 108 -> 27, at
+// 512 rows 111 -> 47; 7168 x 7168 at 61 rows 128 -> 33; 4096 x 4096 at 1024 rows stays whole
+// (256 workgroups, 82 us).
+static int gemm_rows_splits(int mt, int nrows, int K, int O) {
+    const long long tasks = (long long)((nrows + 16 * mt - 1) / (16 * mt)) * (O / 256);
+    const int np = (K / kGemmBK + 1) / 2, slots = mt == 4 ? 256 : 512;
+    const double pair_us = mt == 4 ? 8. : mt == 2 ? 5. : 3.6;
+    const double sum_us = (double)nrows * O * 8 / 4e6;  // 4 TB/s, written and read
+    int best = 1;
+    double least = 0;
+    for (int ks = 1; ks <= np && (size_t)ks * nrows * O * 4 <= kGemmRowsPart; ++ks) {
+        const double us = (double)((tasks * ks + slots - 1) / slots) * ((np + ks - 1) / ks) * pair_us +
+                          (ks > 1 ? 5 + ks * sum_us : 0);
+        if (ks == 1 || us < least)
+            best = ks, least = us;
+    }
+    return best;
+}
+
 hipError_t launch_gemm_rows(int fmt, int terms, int mt, const ExpertWork *ew1, int nrows,
-                            const void *pin, float *out, int K, int O, hipStream_t st) {
+                            const void *pin, float *out, float *part, int K, int O,
+                            hipStream_t st) {
     if (nrows <= 0)
         return hipSuccess;
     if (K % kGemmBK || O % 256 || gemm_lds_bytes(fmt, terms, mt) > 163840 || !ew1)
@@ -872,26 +932,33 @@ hipError_t launch_gemm_rows(int fmt, int terms, int mt, const ExpertWork *ew1, i
     GemmArgs a{};
     a.ew1 = *ew1;
     a.nrows_all = nrows;
+    a.ks = part ? gemm_rows_splits(mt, nrows, K, O) : 1;
     a.pin = static_cast<const __bf16 *>(pin);
-    a.out = out;
+    a.out = a.ks > 1 ? part : out;
     a.nbn = O / 256;
     a.K = K;
     a.O = O;
     a.rcap = nrows;
-    const int n_items = (nrows + 16 * mt - 1) / (16 * mt);
+    const int n_items = (nrows + 16 * mt - 1) / (16 * mt) * a.ks;
     if (terms != 2)
         return hipErrorInvalidValue;
-#define MVLLM_ROWS(F)                                                                          \
-    return mt == 1 ? launch_gemm_t<F, false, 2, 1, true>(a, n_items, st)                      \
-         : mt == 2 ? launch_gemm_t<F, false, 2, 2, true>(a, n_items, st)                      \
-         : mt == 4 ? launch_gemm_t<F, false, 2, 4, true>(a, n_items, st)                      \
-                   : hipErrorInvalidValue
+    hipError_t e = hipErrorInvalidValue;
+#define MVLLM_ROWS(F)                                                                     \
+    e = mt == 1   ? launch_gemm_t<F, false, 2, 1, true>(a, n_items, st)                   \
+        : mt == 2 ? launch_gemm_t<F, false, 2, 2, true>(a, n_items, st)                   \
+        : mt == 4 ? launch_gemm_t<F, false, 2, 4, true>(a, n_items, st)                   \
+                  : hipErrorInvalidValue
     if (fmt == 4)
         MVLLM_ROWS(4);
-    if (fmt == 7)
+    else if (fmt == 7)
         MVLLM_ROWS(7);
 #undef MVLLM_ROWS
-    return hipErrorInvalidValue;
+    if (e != hipSuccess || a.ks == 1)
+        return e;
+    const size_t n4 = (size_t)nrows * O / 4;
+    hipLaunchKernelGGL(k_sum_splits, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st,
+                       reinterpret_cast<const f4v *>(part), reinterpret_cast<f4u *>(out), n4, a.ks);
+    return hipGetLastError();
 }
 
 hipError_t launch_prep_planes(int fmt, int terms, const float *x, const int *rows_map, int R,

@@ -219,9 +219,14 @@ hipError_t launch_gemm_wide(bool dual, const ExpertWork *ew, const void *items, 
                             int act, float act_a, float act_b, hipStream_t st,
                             const int *n_items_dev);
 // One matrix (w[2], s[2] of *ew1) over input rows [0, nrows) of the planes, in items of
-// 16 * mt rows computed in the kernel (a dense linear): out [nrows][O] f32.
+// 16 * mt rows computed in the kernel (a dense linear): out [nrows][O] f32.  Launches of few
+// workgroups split K; the splits' sums go to part (kGemmRowsPart bytes; null: no splits) and
+// are added in order.
+constexpr size_t kGemmRowsPart = size_t(32) << 20;
 hipError_t launch_gemm_rows(int fmt, int terms, int mt, const ExpertWork *ew1, int nrows,
-                            const void *pin, float *out, int K, int O, hipStream_t st);
+                            const void *pin, float *out, float *part, int K, int O,
+                            hipStream_t st);
+
 hipError_t launch_prep_planes(int fmt, int terms, const float *x, const int *rows_map, int R,
                               int K, int rcap, void *planes, hipStream_t st,
                               const int *n_live = nullptr, int src_rows = -1);

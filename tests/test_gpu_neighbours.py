@@ -292,3 +292,25 @@ def test_linear_int8_rows_aligned_to_four_bytes(hip, orc):
     hip.linear_dev(8, raw.data_ptr() + 4, dev(sc), O, K, dev(x), n, y)
     torch.cuda.synchronize()
     assert npref.rel_err(y.cpu().numpy(), orc.matmul(8, x, w, sc)) < TOL_F32
+
+
+@pytest.mark.parametrize("fmt,O,K,n", [(4, 512, 7168, 1), (7, 256, 2304, 17), (4, 256, 2304, 100),
+                                       (7, 512, 6144, 65), (4, 256, 2048, 16), (7, 256, 2048, 17),
+                                       (4, 512, 1024, 32), (7, 256, 512, 64), (4, 256, 512, 65),
+                                       (4, 512, 512, -5), (7, 2304, 2304, -33)])
+def test_linear_splits_against_64_bits(hip, fmt, O, K, n):
+    """K split over workgroups (whole and ragged ranges of step pairs) and the few-row launch on
+    either side of its line; n < 0: y overwrites x.  Two bf16 terms are 2^-17 of each product, the
+    sums' roundings far below it: 1e-5."""
+    rng = np.random.default_rng(O + K + abs(n) + fmt)
+    m = abs(n)
+    x = rng.standard_normal((m, K)).astype(np.float32)
+    e = expert_arrays(rng, fmt, K, O)
+    w = npref.dequant(fmt, e["gp"], e["gs"], K)
+    xd = dev(x)
+    y = xd if n < 0 else torch.zeros((m, O), dtype=torch.float32, device="cuda")
+    for _ in range(2):
+        xd.copy_(dev(x))
+        hip.linear_dev(fmt, dev(e["gp"]), dev(e["gs"]), O, K, xd, m, y)
+        torch.cuda.synchronize()
+        assert npref.rel_err(y.cpu().numpy(), x.astype(np.float64) @ w.astype(np.float64).T) < 1e-5
