@@ -142,7 +142,7 @@ int mvllm_hip_moe_block_dev_noalloc(int nb, int D, int Iinter, int fmt, int qgs,
  * D % 16 == 0, Iinter % 32 == 0, D % 32 == 0 and rows are 16-byte aligned.  Shapes the
  * 256-wide kernels do not take (D or Iinter not a multiple of 256 for fmt 4/7) run on the
  * matrix cores with exact f32 activations (three bf16 terms) when D and Iinter are
- * multiples of 16, weights are 8-byte and int4 scales 4-byte aligned; the rest (odd widths,
+ * multiples of 16 from 64 on, weights are 8-byte and int4 scales 4-byte aligned; the rest (odd widths,
  * odd fmt 0 shapes, misaligned pointers) an exact element-wise f32 kernel. */
 int mvllm_hip_set_option(const char *key, long long value);
 

@@ -17,8 +17,9 @@
 //   FMA applies the group's scale.  (A chain over n from -8 sum x decodes with fewer
 //   instructions, but its cancellation cost accuracy: 2.5e-7 against 1.5e-7 of 64 bits.)
 //   MXFP4: the block's scale is folded into the decode (exact for bytes 2..252).
-// A wave that meets an infinite activation, a non-finite int4 scale or another MXFP4 scale
-// byte forms its sums again element by element, as the reference does.
+// A wave that meets an activation of 2^118 or more (a group's unscaled sum could overflow
+// where the reference's does not), a non-finite int4 scale or another MXFP4 scale byte forms
+// its sums again element by element, as the reference does.
 //
 // Bound by the latency of the loads of the few waves that its registers allow, then by the
 // vector ALU (the split of x, the decode): NT tiles share one split.  24 tokens, 32 int4
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(64 * W) void k_q_rows(QArgs A) {
                     b.x[u][mt][v] = xr[mt][16 * (size_t)k + v];
         }
     };
-    float xmax = 0.f;   // largest |x| met (infinite: the wave's sums are formed again)
+    float xmax = 0.f;   // largest |x| met (2^118 up: the wave's sums are formed again)
     uint32_t exc = 0;   // a scale that the decode does not reproduce
     auto compute = [&] __attribute__((always_inline)) (const Buf &b, int u) {
         __builtin_amdgcn_sched_barrier(0);
@@ -248,7 +249,7 @@ __global__ __launch_bounds__(64 * W) void k_q_rows(QArgs A) {
     }
     // C[4 q + i][t] of row tile mt and tile m -> LDS
     float *mine = red[wave];
-    if (__any(exc != 0 || xmax == INFINITY)) {
+    if (__any(exc != 0 || xmax >= 0x1p118f)) {
         const int k0 = 64 * kb0, k1 = wave == W - 1 ? K : 64 * kb1;
         for (int e = 0; e < MT * NT * 4; ++e) {
             const int mt = e / (4 * NT), m = e / 4 % NT, i = e & 3;
@@ -303,7 +304,9 @@ __global__ __launch_bounds__(64 * W) void k_q_rows(QArgs A) {
     }
 }
 
-bool q_rows_fits(int fmt, int K) { return (fmt == 4 || fmt == 7) && K >= 16 && K % 16 == 0; }
+// K >= 64: the loads before the partial block read a whole 64-wide one (rows of fewer elements
+// end before lane q's 16 of it).
+bool q_rows_fits(int fmt, int K) { return (fmt == 4 || fmt == 7) && K >= 64 && K % 16 == 0; }
 
 hipError_t launch_q_rows(int fmt, bool dual, int mt, const ExpertWork *ew, const void *items,
                          int n_items, const ExpertWork *ew1, int nrows_all, const float *in,

@@ -256,7 +256,7 @@ hipError_t launch_rmsnorm(const float *x, const float *w, float *y, int rows, in
 
 // int4 / MXFP4 matrices of any width with exact f32 activations (kern_qrows.hip): items,
 // ew1, in_rows, mi and the outputs as launch_f32mm's (dual H and single Y are f32 rows).
-// Requires K % 16 == 0 (q_rows_fits), 16-byte aligned input rows, 8-byte aligned weights
+// Requires K % 16 == 0 and K >= 64 (q_rows_fits), 16-byte aligned input rows, 8-byte aligned weights
 // and 4-byte aligned int4 scales; any O.
 bool q_rows_fits(int fmt, int K);
 hipError_t launch_q_rows(int fmt, bool dual, int mt, const ExpertWork *ew, const void *items,

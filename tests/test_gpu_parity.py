@@ -202,10 +202,16 @@ DEV_CASES = [
     (0, 64, 48, [2, 1], 3, 1, 3.0, 0.0, (0,), 0),                  # f32 weights
     (4, 2048, 1024, [7, 1, 13], 16, 1, 7.0, 0.0, (), 0),           # rows > one item
     (7, 2048, 1024, [5, 9], 12, 2, 4.0, 25.0, (), 0),
-    # widths that are no multiples of 256: partial 64-blocks of K (16, 32, 48), O past a tile,
-    # 16- and 32-row items, an empty expert, skips
+]
+
+# widths that are no multiples of 256: partial 64-blocks of K (16, 32, 48), one whole block, O
+# past a tile, 16- and 32-row items, an empty expert, skips; below 64 the element-wise kernel
+WIDTH_CASES = [
     (4, 16, 48, [1], 1, 0, 0.0, 0.0, (), 0),
     (7, 48, 16, [3], 3, 2, 4.0, 25.0, (), 0),
+    (4, 64, 32, [1], 1, 0, 0.0, 0.0, (), 0),
+    (4, 64, 80, [1], 1, 0, 0.0, 0.0, (), 0),
+    (7, 96, 64, [3], 3, 2, 4.0, 25.0, (), 0),
     (4, 208, 176, [17, 16, 33], 40, 1, 7.0, 0.0, (), 2),
     (7, 2080, 1056, [1, 0, 33, 16], 40, 2, 4.0, 25.0, (2,), 1),
     (4, 2112, 704, [2] * 24, 12, 0, 0.0, 0.0, (), 0),              # four-tile waves
@@ -231,7 +237,7 @@ def test_moe_block_bf16_mode(hip, orc, case):
     assert err < 1e-2
 
 
-@pytest.mark.parametrize("case", DEV_CASES)
+@pytest.mark.parametrize("case", DEV_CASES + WIDTH_CASES)
 def test_moe_block_dev_parity(hip, orc, case):
     fmt, D, I, nr, S, act, a, b, nulls, bad = case
     say("moe_block_dev", case)
@@ -343,6 +349,22 @@ def test_nonfinite_propagation(hip, orc, D, I):
         fin = np.isfinite(exp)
         assert np.array_equal(np.sign(got[np.isinf(exp)]), np.sign(exp[np.isinf(exp)]))
         assert npref.rel_err(got[fin], exp[fin]) < TOL_F32
+
+
+@pytest.mark.parametrize("D,I", [(250, 130), (560, 304)])
+def test_large_activations_small_scales(hip, orc, D, I):
+    """Activations near 2^121 against int4 scales near 2^-124: finite in the reference, though
+    a sum over unscaled codes overflows; on the element-wise path and the one for other widths."""
+    say("large activations", D, I)
+    rng = np.random.default_rng(D)
+    c = random_case(rng, 4, D, I, [2, 1], 3, 0, 0.0, 0.0)
+    c.xg *= np.float32(2.0 ** 121)
+    for s in c.gs + c.us:
+        s *= np.float32(2.0 ** -118)
+    got = run_dev(hip, c, 0, 0.0, 0.0)
+    exp = oracle_out(orc, c, 0, 0.0, 0.0)
+    assert np.isfinite(exp).all()
+    assert npref.rel_err(got, exp) < TOL_F32
 
 
 @pytest.mark.parametrize("fmt", [4, 7])
