@@ -208,6 +208,189 @@ __global__ __launch_bounds__(64 * W) void k_f32mm_rows(F32Args A) {
     }
 }
 
+// Many rows: 64 input rows x 16 NB weight rows a workgroup, through LDS.  The kernel above
+// reads 64 bytes of each row at a time straight into the operands, for half the output tile
+// and eight times over the waves of K: the requests, not the matrix cores, set its pace.  Here
+// a K step of 32 is a whole line of every row, read once for the four waves that share it, two
+// steps ahead (registers, then one of two LDS buffers; 16-byte chunks XOR-swizzled by the
+// row, so that eight rows' reads of one chunk lie in different banks); wave w multiplies row
+// tile w with all NB weight tiles.  int8 codes convert to f32 as they are staged.  Two such
+// groups of four waves split K and add at the end: with one, a CU that has a single workgroup
+// waits on its loads (1024 x 7168 at 512 rows 112 us, 91 with two).  Each 512 of K sum in
+// their own chain, which then adds to the total: no less exact than eight waves' split.
+// The f32 expert of 6144 x 2048 over 300 rows 386 -> 291 us per call (59 -> 78 TFLOP/s), f32
+// 7168 x 7168 over 1024 rows 1178 -> 964 us (109 of the f32 matrix cores' 157 TFLOP/s), int8
+// 1116 -> 963 us.  Bound by the matrix cores where the workgroups fill whole rounds.
+template <bool DUAL, int NB, int WK>
+__global__ __launch_bounds__(512) void k_f32mm_tile(F32Args A) {
+    constexpr int BK = 32, XC = 64 * BK / 4 / 256;      // chunks of x a thread stages
+    constexpr int WC = 16 * NB * BK / 4 / 256;          // and of the weights
+    constexpr int CT = DUAL ? NB / 2 : NB;              // output column tiles
+    static_assert(NB % 2 == 0 && WC >= 1, "weight tiles in pairs");
+    __shared__ float4 lx[2][2][64 * BK / 4];
+    __shared__ float4 lw[2][2][16 * NB * BK / 4];
+    const int task = xcd_task(blockIdx.x, A.n_tasks);
+    const int cb = task / A.n_items, item = task - cb * A.n_items;
+    const int tid = threadIdx.x & 255;
+    const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto &sx = lx[grp];
+    auto &sw = lw[grp];
+    const int lane = tid & 63, t = lane & 15, q = lane >> 4;
+    const int K = A.K, O = A.O, col0 = cb * 16 * CT;
+    F32Item it;
+    if (A.items) {
+        it = A.items[item];
+    } else {
+        it.a = 0;
+        it.r0 = item * 64;
+        it.nrow = min(64, A.nrows_all - it.r0);
+    }
+    const ExpertWork &ew = A.items ? A.ew[it.a] : A.ew1;
+    const int jbase = ew.row0 + it.r0;
+    // this thread's chunks: chunk tid % 8 of rows tid / 8 + 32 j (rows past the item or the
+    // matrix repeat the last; their results are not stored)
+    const int c = tid & 7, r0 = tid >> 3;
+    const float *xr[XC];
+#pragma unroll
+    for (int j = 0; j < XC; ++j) {
+        const int r = min(r0 + 32 * j, it.nrow - 1);
+        const int src = A.in_rows ? A.in_rows[jbase + r] : jbase + r;
+        xr[j] = A.in + (size_t)src * K;
+    }
+    const char *wr[WC];
+#pragma unroll
+    for (int j = 0; j < WC; ++j) {
+        const int r = r0 + 32 * j, m = r >> 4;
+        const int row = min(col0 + 16 * (m % CT) + (r & 15), O - 1);
+        const char *w = static_cast<const char *>(ew.w[DUAL ? m / CT : A.mi]);
+        wr[j] = w + (size_t)row * (size_t)K * (WK ? 1 : 4);
+    }
+    struct Stage {
+        float4 x[XC];
+        u32x4 w[WC];  // int8: word 0 only
+    };
+    // this group's K steps: [s0, s0 + ns); the second group's may end past K
+    const int ns = ((K + BK - 1) / BK + 1) / 2, s0 = grp * ns;
+    auto load = [&] __attribute__((always_inline)) (Stage &b, int s) {
+        const int k = (s0 + min(s, ns - 1)) * BK + 4 * c;
+        const int kc = min(k, K - 4);  // past K: zeros (set at the store)
+#pragma unroll
+        for (int j = 0; j < WC; ++j) {
+            if constexpr (WK)
+                b.w[j].x = *reinterpret_cast<const uint32_t *>(wr[j] + kc);
+            else
+                b.w[j] = *reinterpret_cast<const u32x4 *>(wr[j] + 4 * (size_t)kc);
+        }
+#pragma unroll
+        for (int j = 0; j < XC; ++j)
+            b.x[j] = *reinterpret_cast<const float4 *>(xr[j] + kc);
+    };
+    auto store = [&] __attribute__((always_inline)) (const Stage &b, int s, int buf) {
+        const bool in = s < ns && (s0 + s) * BK + 4 * c < K;
+        const int at = 8 * r0 + (c ^ (r0 & 7));  // rows 32 apart swizzle alike
+#pragma unroll
+        for (int j = 0; j < XC; ++j)
+            sx[buf][at + 256 * j] = in ? b.x[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int j = 0; j < WC; ++j) {
+            float4 w;
+            if constexpr (WK)
+                w = make_float4((float)(int8_t)b.w[j].x, (float)(int8_t)(b.w[j].x >> 8),
+                                (float)(int8_t)(b.w[j].x >> 16), (float)(int8_t)(b.w[j].x >> 24));
+            else
+                w = __builtin_bit_cast(float4, b.w[j]);
+            sw[buf][at + 256 * j] = in ? w : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    f4v acc[NB], tot[NB];
+#pragma unroll
+    for (int m = 0; m < NB; ++m)
+        acc[m] = tot[m] = f4v{0.f, 0.f, 0.f, 0.f};
+    const bool live = 16 * wave < it.nrow;
+    auto mma = [&] __attribute__((always_inline)) (int buf) {
+        if (!live)  // wave-uniform: a row tile past the item
+            return;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int at = 8 * t + ((4 * h + q) ^ (t & 7));
+            const float4 x = sx[buf][128 * wave + at];
+            float4 w[NB];
+#pragma unroll
+            for (int m = 0; m < NB; ++m)
+                w[m] = sw[buf][128 * m + at];
+#pragma unroll
+            for (int m = 0; m < NB; ++m)
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, w[m].x, acc[m], 0, 0, 0);
+#pragma unroll
+            for (int m = 0; m < NB; ++m)
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, w[m].y, acc[m], 0, 0, 0);
+#pragma unroll
+            for (int m = 0; m < NB; ++m)
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, w[m].z, acc[m], 0, 0, 0);
+#pragma unroll
+            for (int m = 0; m < NB; ++m)
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, w[m].w, acc[m], 0, 0, 0);
+        }
+    };
+    auto fold = [&] __attribute__((always_inline)) () {
+#pragma unroll
+        for (int m = 0; m < NB; ++m) {
+            tot[m] += acc[m];
+            acc[m] = f4v{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    // step s: LDS buffer s & 1; its successor waits in one register set while the one after it
+    // is loaded into the other.  One barrier a step: the buffer that a step writes was last
+    // read before the barrier that ended the step before.
+    Stage g0, g1;
+    load(g0, 0);
+    load(g1, 1);
+    store(g0, 0, 0);
+    __syncthreads();
+    for (int s = 0; s < ns; s += 2) {
+        load(g0, s + 2);
+        mma(0);
+        store(g1, s + 1, 1);  // past the last step: zeros
+        __syncthreads();
+        load(g1, s + 3);
+        mma(1);
+        store(g0, s + 2, 0);
+        if ((s & 14) == 14)
+            fold();
+        __syncthreads();
+    }
+    fold();
+    // the second group's sums are added to the first's
+    f4v *part = reinterpret_cast<f4v *>(&lx[0][0][0]);  // 256 NB of its 2048 chunks
+    if (grp)
+#pragma unroll
+        for (int m = 0; m < NB; ++m)
+            part[256 * m + tid] = tot[m];
+    __syncthreads();
+    if (grp)
+        return;
+#pragma unroll
+    for (int m = 0; m < NB; ++m)
+        tot[m] += part[256 * m + tid];
+    // C[4 q + i][t] of row tile `wave` and weight tile m
+#pragma unroll
+    for (int m = 0; m < CT; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 16 * wave + 4 * q + i, col = col0 + 16 * m + t;
+            if (r >= it.nrow || col >= O)
+                continue;
+            float *dst = A.out + (size_t)(jbase + r) * O + col;
+            if constexpr (DUAL)
+                *dst = mf_act(A.act, tot[m][i], tot[m + CT][i], A.act_a, A.act_b);
+            else if constexpr (WK != kRowsF32)
+                *dst = tot[m][i] * static_cast<const float *>(ew.s[A.mi])[col];
+            else
+                *dst = tot[m][i];
+        }
+}
+
 bool f32mm_fits(bool dual, int K, int O) {
     return K >= 16 && K % 16 == 0 && O % (dual ? 16 : 32) == 0;
 }
@@ -241,6 +424,35 @@ hipError_t launch_f32mm(bool dual, int mt, const ExpertWork *ew, const void *ite
     if (n_items <= 0)
         return hipSuccess;
     a.n_items = n_items;
+    // Blocks of 64 rows through LDS where they are more than a workgroup a CU (at 256 of them:
+    // int8 1024 x 7168 at 512 rows 91 us against 82 of the rows' kernel, f32 91 against 88; at
+    // 320, 2048 x 6144 at 300 rows, 128 against 144, int8 128 against 137).  Four weight tiles
+    // a workgroup where their rounds of 256 cost no more than those of two.
+    if (mt == 4 && !out2) {
+        const auto tasks = [&](int nb) {
+            const int cw = dual ? 8 * nb : 16 * nb;
+            return (long long)n_items * ((O + cw - 1) / cw);
+        };
+        const long long t2 = tasks(2), t4 = tasks(4);
+        if (t2 > 256) {
+            const bool four = (t4 + 255) / 256 * 2 <= (t2 + 255) / 256;
+            a.n_tasks = (int)(four ? t4 : t2);
+            const dim3 grid((unsigned)a.n_tasks), block(512);
+#define MVLLM_F32T(D, I)                                                                  \
+    do {                                                                                  \
+        if (four) hipLaunchKernelGGL((k_f32mm_tile<D, 4, I>), grid, block, 0, st, a);     \
+        else hipLaunchKernelGGL((k_f32mm_tile<D, 2, I>), grid, block, 0, st, a);          \
+    } while (0)
+            if (dual)
+                MVLLM_F32T(true, kRowsF32);
+            else if (i8)
+                MVLLM_F32T(false, kRowsI8x4);
+            else
+                MVLLM_F32T(false, kRowsF32);
+#undef MVLLM_F32T
+            return hipGetLastError();
+        }
+    }
     const bool wide8 = i8 && K % 64 == 0 && ew1 && (reinterpret_cast<uintptr_t>(ew1->w[mi]) & 15) == 0;
     // Two tiles a wave read the input rows once for twice the weights; one tile a wave gives
     // twice the workgroups.  Two from 448 one-tile tasks on (the 256 CUs then have about a

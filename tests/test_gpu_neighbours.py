@@ -64,6 +64,8 @@ F32_CASES = [
     (32, 16, [1], 1, 0, 0.0, 0.0),                  # one K block, one tile
     (4128, 272, [17, 16], 40, 1, 7.0, 0.0),         # K of unequal wave ranges, 8-column tiles
     (4160, 3600, [2], 2, 2, 4.0, 25.0),             # 16-column dual tiles, 16 waves
+    (96, 2064, [64, 64, 33], 70, 2, 4.0, 25.0),     # 64-row blocks, 4 weight tiles, ragged columns
+    (1056, 2064, [130, 64, 40], 150, 1, 7.0, 0.0),  # 64-row blocks, 2 weight tiles, chains of 512
 ]
 
 
@@ -132,7 +134,9 @@ def test_router_matches_host_router(hip, orc, T, D, E, k, rscale, bias):
                                        (8, 2048, 7168, 1), (8, 7168, 2048, 4),
                                        (8, 7168, 7168, 1), (8, 96, 48, 37),
                                        (0, 32, 16, 1), (0, 480, 1040, 17), (0, 7200, 4112, 16),
-                                       (8, 160, 4160, 33), (8, 7200, 4096, 2), (8, 32, 80, 65)])
+                                       (8, 160, 4160, 33), (8, 7200, 4096, 2), (8, 32, 80, 65),
+                                       (0, 4128, 80, 129), (0, 4128, 16, 300), (0, 4128, 1040, 300),
+                                       (8, 4128, 144, 129), (8, 4128, 1040, 257)])
 def test_linear(hip, orc, fmt, O, K, n):
     """fmt 8 (QuantMat's int8 rows, MVLLM_DENSE_BITS=8) at K3's latent shapes, with codes
     and scales from the reference's quantizer rule (row amax / 127, clamp +-127) and an
