@@ -208,9 +208,9 @@ __global__ __launch_bounds__(64 * W) void k_f32mm_rows(F32Args A) {
     }
 }
 
-// Many rows: 64 input rows x 16 NB weight rows a workgroup, through LDS.  The kernel above
-// reads 64 bytes of each row at a time straight into the operands, for half the output tile
-// and eight times over the waves of K: the requests, not the matrix cores, set its pace.  Here
+// Many rows: 64 input rows x 16 NB weight rows a workgroup, through LDS.  In the kernel above
+// each wave reads 64 bytes, half a line, of 96 rows for 32 matrix instructions, and the waves
+// of a workgroup read different parts of K, so nothing is shared.  Here
 // a K step of 32 is a whole line of every row, read once for the four waves that share it, two
 // steps ahead (registers, then one of two LDS buffers; 16-byte chunks XOR-swizzled by the
 // row, so that eight rows' reads of one chunk lie in different banks); wave w multiplies row
