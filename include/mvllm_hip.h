@@ -253,8 +253,8 @@ int mvllm_hip_router_dev(const float *x, const float *w, const float *bias, int 
  * (quant::matmul_int8_row, src/quant/quant.cpp:255-268; MVLLM_DENSE_BITS=8), each code
  * exact in f32 on the f32 matrix cores and the row scale applied once to the finished
  * sum (K % 16, O % 32, 4-byte aligned codes and scales, 16-byte aligned x).  Calls on
- * one stream, or ordered by the caller: the int4 / MXFP4 forms share one input buffer
- * (a call on another stream than the previous one waits for it). */
+ * one stream, or ordered by the caller; the int4 / MXFP4 forms share scratch, so such a call
+ * on another stream than the previous call's waits for that call, and later calls for it. */
 int mvllm_hip_linear_dev(int fmt, const void *w, const void *scales, int O, int K,
                          const float *x, int n, float *y, void *stream);
 

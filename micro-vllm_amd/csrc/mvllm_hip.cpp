@@ -2533,6 +2533,11 @@ int mvllm_hip_linear_dev(int fmt, const void *w, const void *scales, int O, int 
     const int terms = 2;
     HIP_TRY(C.Lp.ensure((size_t)terms * 2 * n * K));
     HIP_TRY(C.Ls.ensure(kGemmRowsPart));
+    // A call on another stream than the previous one waits for it, as the block entry points'
+    // do: the planes buffer is shared by every call, and the form a call takes depends on its
+    // sizes and addresses, on which its order against other calls must not.
+    if (!order_after_previous(C, st))
+        return 0;
     // Few rows of a short K: one launch on the f32 rows themselves, where the planes, the GEMM
     // and the sum of its splits are three (7168 x 512 at 1 row 9.2 -> 6.0 us, at 32 rows 11.5
     // -> 6.8; 7168 x 1024 at 16 rows 13.0 -> 9.9, 7168 x 2048 at 1 row 12.8 -> 11.0; equal at
@@ -2540,20 +2545,16 @@ int mvllm_hip_linear_dev(int fmt, const void *w, const void *scales, int O, int 
     // which the planes allow: its workgroups read x while others write y.
     const uintptr_t xb = reinterpret_cast<uintptr_t>(x), yb = reinterpret_cast<uintptr_t>(y);
     const bool apart = xb + (size_t)n * K * 4 <= yb || yb + (size_t)n * O * 4 <= xb;
-    if ((long long)K * ((n + 15) / 16) <= 2048 && apart && aligned(x, 16) && q_rows_fits(fmt, K)) {
+    if ((long long)K * ((n + 15) / 16) <= 2048 && apart && aligned(x, 16)) {
         HIP_TRY(launch_q_rows(fmt, false, n <= 16 ? 1 : 2, nullptr, nullptr, 0, &ew, n, x, nullptr,
                               y, 2, K, O, 0, 0.f, 0.f, st));
-        return 1;
+    } else {
+        // the input rows as two bf16 terms (2^-17 relative), then the grouped GEMM
+        HIP_TRY(launch_prep_planes(fmt, terms, x, nullptr, n, K, n, C.Lp.p, st));
+        const int mt = n <= 16 ? 1 : n <= 32 ? 2 : 4;
+        HIP_TRY(launch_gemm_rows(fmt, terms, mt, &ew, n, C.Lp.p, y, static_cast<float *>(C.Ls.p),
+                                 K, O, st));
     }
-    // the input rows as two bf16 terms (2^-17 relative), then the grouped GEMM.  The planes
-    // buffer is shared by every call: a call on another stream than the previous one waits for
-    // it first, as the block entry points do.
-    if (!order_after_previous(C, st))
-        return 0;
-    HIP_TRY(launch_prep_planes(fmt, terms, x, nullptr, n, K, n, C.Lp.p, st));
-    const int mt = n <= 16 ? 1 : n <= 32 ? 2 : 4;
-    HIP_TRY(launch_gemm_rows(fmt, terms, mt, &ew, n, C.Lp.p, y, static_cast<float *>(C.Ls.p), K, O,
-                             st));
     C.last_stream = st;
     C.have_last = true;
     return 1;

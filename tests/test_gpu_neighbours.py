@@ -318,3 +318,37 @@ def test_linear_splits_against_64_bits(hip, fmt, O, K, n):
         hip.linear_dev(fmt, dev(e["gp"]), dev(e["gs"]), O, K, xd, m, y)
         torch.cuda.synchronize()
         assert npref.rel_err(y.cpu().numpy(), x.astype(np.float64) @ w.astype(np.float64).T) < 1e-5
+
+
+@pytest.mark.parametrize("fmt", [4, 7])
+def test_linears_wait_across_streams(hip, fmt):
+    """An int4 / MXFP4 linear waits for the library's previous call on another stream, in
+    every form it takes: planes (100 rows) -> few rows -> planes -> few rows, each on a stream
+    of its own and reading the one before it, with a long product ahead of the first.  Equal
+    bits to the same chain on one stream."""
+    rng = np.random.default_rng(600 + fmt)
+    shapes = [(512, 2048, 100), (2048, 512, 16), (512, 2048, 40), (256, 512, 8)]  # O, K, rows
+    ws = [expert_arrays(rng, fmt, K, O) for O, K, _ in shapes]
+    ws = [(dev(e["gp"]), dev(e["gs"])) for e in ws]
+    x0 = dev(rng.standard_normal((100, 2048)).astype(np.float32))
+    big = torch.randn(4096, 4096, device="cuda")
+
+    def chain(streams):
+        # a linear's input: the first K floats of each of its rows lie in the last output
+        bufs = [x0] + [torch.zeros(100 * 2048, device="cuda") for _ in shapes]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            p = big
+            for _ in range(40):
+                p = p @ big
+        for i, (O, K, n) in enumerate(shapes):
+            hip.linear_dev(fmt, *ws[i], O, K, bufs[i], n, bufs[i + 1], stream=streams[i])
+        torch.cuda.synchronize()
+        return [b.cpu().numpy() for b in bufs[1:]]
+
+    s = [torch.cuda.Stream() for _ in shapes]
+    exp = chain([s[0]] * len(shapes))
+    got = chain(s)
+    assert all(np.abs(e).max() > 0 for e in exp)
+    for g, e in zip(got, exp):
+        assert np.array_equal(g.view(np.uint32), e.view(np.uint32))
