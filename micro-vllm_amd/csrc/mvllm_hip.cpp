@@ -426,6 +426,11 @@ void build_plan(Plan &P, int nb, int D, int Iinter, int fmt, const void *const *
 
 bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 
+bool overlap(const void *p, size_t n, const void *q, size_t m) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+    return a < b + m && b < a + n;
+}
+
 // Does the decode kernel take this phase shape (K split ks, nt tiles per wave)?
 bool dec_fits(int fmt, int K, int O, int rmax, int terms, bool dual, int ks, int nt) {
     const int tiles_wg = (kDecWaves / ks) * (dual ? 1 : nt);
@@ -2484,7 +2489,14 @@ int mvllm_hip_router_dev(const float *x, const float *w, const float *bias, int 
     };
     while (mt < 4 && tasks() > 256)
         mt *= 2;
-    float *half2 = split && tasks() <= 256 ? choice : nullptr;
+    // The second half's sums are written while other workgroups read x and w and write
+    // scores, so only a choice workspace of its own takes them (without the split choice is
+    // written after the last read: one buffer may serve as both workspaces, or x's memory).
+    const size_t ch = (size_t)n_tok * n_exp * 4;
+    const bool own = !overlap(choice, ch, scores, ch) &&
+                     !overlap(choice, ch, x, (size_t)n_tok * D * 4) &&
+                     !overlap(choice, ch, w, (size_t)n_exp * D * 4);
+    float *half2 = split && tasks() <= 256 && own ? choice : nullptr;
     HIP_TRY(launch_f32mm(false, mt, nullptr, nullptr, 0, &ew, n_tok, x, nullptr, scores, 0, D,
                          n_exp, 0, 0.f, 0.f, st, false, half2));
     if (fused) {
@@ -2543,8 +2555,7 @@ int mvllm_hip_linear_dev(int fmt, const void *w, const void *scales, int O, int 
     // -> 6.8; 7168 x 1024 at 16 rows 13.0 -> 9.9, 7168 x 2048 at 1 row 12.8 -> 11.0; equal at
     // 2048 and 16 rows, behind past it: 6144 at 1 row 14.6 -> 19.6).  Not where y overlaps x,
     // which the planes allow: its workgroups read x while others write y.
-    const uintptr_t xb = reinterpret_cast<uintptr_t>(x), yb = reinterpret_cast<uintptr_t>(y);
-    const bool apart = xb + (size_t)n * K * 4 <= yb || yb + (size_t)n * O * 4 <= xb;
+    const bool apart = !overlap(x, (size_t)n * K * 4, y, (size_t)n * O * 4);
     if ((long long)K * ((n + 15) / 16) <= 2048 && apart && aligned(x, 16)) {
         HIP_TRY(launch_q_rows(fmt, false, n <= 16 ? 1 : 2, nullptr, nullptr, 0, &ew, n, x, nullptr,
                               y, 2, K, O, 0, 0.f, 0.f, st));

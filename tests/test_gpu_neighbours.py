@@ -128,6 +128,35 @@ def test_router_matches_host_router(hip, orc, T, D, E, k, rscale, bias):
                   np.maximum(np.abs(ew_s[agree]), 1e-30)) < 1e-5
 
 
+@pytest.mark.parametrize("T,D,E,k", [(1, 7168, 384, 8), (61, 2048, 256, 6), (300, 2048, 64, 4)])
+@pytest.mark.parametrize("shared", ["scores", "x"])
+def test_router_workspace_shared(hip, T, D, E, k, shared):
+    """choice in the memory of scores (no bias: both hold the mix) or of x, which is read
+    before choice is written: the result of separate workspaces.  The split of K changes the
+    sums' order only: a score by some 1e-6, and a pick where two choices are that close."""
+    rng = np.random.default_rng(T + D + E)
+    x = rng.standard_normal((T, D)).astype(np.float32)
+    w = (rng.standard_normal((E, D)) / np.sqrt(D)).astype(np.float32)
+    f32 = dict(dtype=torch.float32, device="cuda")
+    wd, res = dev(w), []
+    for own in (True, False):
+        xd, scores = dev(x), torch.empty((T, E), **f32)
+        choice = torch.empty((T, E), **f32) if own else scores if shared == "scores" else xd
+        idx, wt = torch.empty((T, k), dtype=torch.int32, device="cuda"), torch.empty((T, k), **f32)
+        hip.router_dev(xd, wd, None, T, D, E, k, 1.0, scores, choice, idx, wt)
+        torch.cuda.synchronize()
+        res.append((idx.cpu().numpy(), wt.cpu().numpy(), scores.cpu().numpy()))
+    mix = 1.0 / (1.0 + np.exp(-(x.astype(np.float64) @ w.astype(np.float64).T)))
+    srt = -np.sort(-mix, axis=1)
+    clear = np.all((srt[:, :k] - srt[:, 1:k + 1]) / srt[:, :k] > 1e-5, axis=1)
+    assert clear.any()
+    for idx, wt, scores in res:
+        assert np.max(np.abs(scores - mix) / mix) < 1e-5
+        assert np.array_equal(idx[clear], np.argsort(-mix, axis=1)[clear, :k])
+        exp = srt[:, :k] / srt[:, :k].sum(axis=1, keepdims=True)
+        assert np.max(np.abs(wt - exp) / exp) < 1e-5
+
+
 @pytest.mark.parametrize("fmt,O,K,n", [(0, 2048, 7168, 1), (0, 7168, 2048, 5), (0, 64, 48, 3),
                                        (4, 2048, 6144, 1), (4, 512, 1024, 40),
                                        (7, 7168, 2048, 3), (7, 256, 512, 70),
