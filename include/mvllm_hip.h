@@ -254,7 +254,10 @@ int mvllm_hip_router_dev(const float *x, const float *w, const float *bias, int 
  * exact in f32 on the f32 matrix cores and the row scale applied once to the finished
  * sum (K % 16, O % 32, 4-byte aligned codes and scales, 16-byte aligned x).  Calls on
  * one stream, or ordered by the caller; the int4 / MXFP4 forms share scratch, so such a call
- * on another stream than the previous call's waits for that call, and later calls for it. */
+ * on another stream than the previous call's waits for that call, and later calls for it.
+ * Their K is split over workgroups where the launch would leave the chip idle; the first such
+ * call allocates 32 MiB for the partial sums (without it, or captured before any such call, a
+ * call runs unsplit). */
 int mvllm_hip_linear_dev(int fmt, const void *w, const void *scales, int O, int K,
                          const float *x, int n, float *y, void *stream);
 

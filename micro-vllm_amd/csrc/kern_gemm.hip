@@ -906,7 +906,7 @@ __global__ __launch_bounds__(256) void k_sum_splits(const f4v *part, f4u *y, siz
 // planes, unsplit -> split: int4 2048 x 6144 at 1 row 51 -> 15 us, at 100 rows 108 -> 27, at
 // 512 rows 111 -> 47; 7168 x 7168 at 61 rows 128 -> 33; 4096 x 4096 at 1024 rows stays whole
 // (256 workgroups, 82 us).
-static int gemm_rows_splits(int mt, int nrows, int K, int O) {
+int gemm_rows_splits(int mt, int nrows, int K, int O) {
     const long long tasks = (long long)((nrows + 16 * mt - 1) / (16 * mt)) * (O / 256);
     const int np = (K / kGemmBK + 1) / 2, slots = mt == 4 ? 256 : 512;
     const double pair_us = mt == 4 ? 8. : mt == 2 ? 5. : 3.6;

@@ -1988,6 +1988,19 @@ int routed_dec(Ctx &C, int D, int I, int fmt, const void *const *table, int n_ta
     return 1;
 }
 
+// The workspace of a dense linear's K splits, allocated by the first call that splits; null
+// where it cannot be (no memory left, or a captured call before any that split): the call then
+// runs unsplit, as it did without the workspace.
+float *splits_buffer(Ctx &C, hipStream_t st) {
+    if (!C.Ls.p) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+            C.Ls.ensure(kGemmRowsPart) != hipSuccess)
+            (void)hipGetLastError();
+    }
+    return static_cast<float *>(C.Ls.p);
+}
+
 }  // namespace
 
 extern "C" {
@@ -2544,7 +2557,6 @@ int mvllm_hip_linear_dev(int fmt, const void *w, const void *scales, int O, int 
     ew.s[2] = scales;
     const int terms = 2;
     HIP_TRY(C.Lp.ensure((size_t)terms * 2 * n * K));
-    HIP_TRY(C.Ls.ensure(kGemmRowsPart));
     // A call on another stream than the previous one waits for it, as the block entry points'
     // do: the planes buffer is shared by every call, and the form a call takes depends on its
     // sizes and addresses, on which its order against other calls must not.
@@ -2563,7 +2575,8 @@ int mvllm_hip_linear_dev(int fmt, const void *w, const void *scales, int O, int 
         // the input rows as two bf16 terms (2^-17 relative), then the grouped GEMM
         HIP_TRY(launch_prep_planes(fmt, terms, x, nullptr, n, K, n, C.Lp.p, st));
         const int mt = n <= 16 ? 1 : n <= 32 ? 2 : 4;
-        HIP_TRY(launch_gemm_rows(fmt, terms, mt, &ew, n, C.Lp.p, y, static_cast<float *>(C.Ls.p),
+        HIP_TRY(launch_gemm_rows(fmt, terms, mt, &ew, n, C.Lp.p, y,
+                                 gemm_rows_splits(mt, n, K, O) > 1 ? splits_buffer(C, st) : nullptr,
                                  K, O, st));
     }
     C.last_stream = st;

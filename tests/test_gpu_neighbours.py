@@ -381,3 +381,48 @@ def test_linears_wait_across_streams(hip, fmt):
     assert all(np.abs(e).max() > 0 for e in exp)
     for g, e in zip(got, exp):
         assert np.array_equal(g.view(np.uint32), e.view(np.uint32))
+
+
+def test_linear_splits_workspace(hip):
+    """The 32 MiB of the K splits are allocated by the first call that splits, not by one that
+    does not need them; a capture before that call runs unsplit, replays give the same bits
+    between eager work, and the split call agrees with 64 bits as well."""
+    rng = np.random.default_rng(77)
+    free = lambda: torch.cuda.mem_get_info()[0]  # noqa: E731
+    mats = {}
+    for O, K in ((512, 1024), (512, 7168), (256, 256)):
+        e = expert_arrays(rng, 4, K, O)
+        mats[O, K] = dev(e["gp"]), dev(e["gs"]), npref.dequant(4, e["gp"], e["gs"], K)
+    xs = rng.standard_normal((3, 1, 7168)).astype(np.float32)
+    few, x = dev(rng.standard_normal((32, 1024)).astype(np.float32)), dev(xs[0])
+    out, y = torch.zeros((32, 512), device="cuda"), torch.zeros((1, 512), device="cuda")
+    inplace = torch.ones((1, 256), device="cuda")
+    w, s, w64 = mats[512, 7168]
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    hip.lib().mvllm_hip_shutdown()
+    hip.init(0)
+    before = free()
+    hip.linear_dev(4, *mats[512, 1024][:2], 512, 1024, few, 32, out, stream=st)   # few rows
+    hip.linear_dev(4, *mats[256, 256][:2], 256, 256, inplace, 1, inplace, stream=st)  # one K step
+    torch.cuda.synchronize()
+    assert before - free() < 16 << 20
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        hip.linear_dev(4, w, s, 512, 7168, x, 1, y, stream=st)
+    seen = []
+    for i in (0, 1, 2, 0):
+        x.copy_(dev(xs[i]))
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        seen.append(y.cpu().numpy())
+        assert npref.rel_err(seen[-1], xs[i].astype(np.float64) @ w64.astype(np.float64).T) < 1e-5
+        hip.linear_dev(4, *mats[512, 1024][:2], 512, 1024, few, 32, out, stream=st)
+    assert np.array_equal(seen[0], seen[3])
+    before = free()
+    hip.linear_dev(4, w, s, 512, 7168, x, 1, y, stream=st)
+    torch.cuda.synchronize()
+    assert before - free() >= 32 << 20
+    assert npref.rel_err(y.cpu().numpy(), xs[0].astype(np.float64) @ w64.astype(np.float64).T) < 1e-5
