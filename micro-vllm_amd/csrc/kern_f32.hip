@@ -33,6 +33,7 @@ struct F32Args {
     float *out2;            // the second half of K's sums when K is split (ksl = 1)
     int mi;                 // single: which matrix of the expert (2 = down; 0 = a linear)
     int n_items, ksl;       // items; log2 of the K splits across workgroups (0 or 1)
+    int nbn;                // k_f32mm_wave: workgroups per item
     int n_tasks, K, O;
     int act;
     float act_a, act_b;
@@ -391,8 +392,176 @@ __global__ __launch_bounds__(512) void k_f32mm_tile(F32Args A) {
         }
 }
 
+constexpr int kF32Waves = 4;
+
+// Short K, or more column tiles than the chip holds workgroups: a wave of its own for each tile
+// of 16 MT rows x 32 columns (dual: 16) over all of K.  The splits above then start eight waves
+// and meet in LDS for a few blocks each.  int8 codes come as 4 of each 16-wide block.  FOLD
+// (K > 512): each 256 of K sum in their own chain, which then adds to the total.
+template <bool DUAL, int MT, bool I8, bool FOLD>
+__global__ __launch_bounds__(64 * kF32Waves) void k_f32mm_wave(F32Args A) {
+    static_assert(!(I8 && DUAL), "int8 rows: single projections only");
+    const int item = blockIdx.x / A.nbn;
+    const int nb = blockIdx.x - item * A.nbn;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, t = lane & 15, q = lane >> 4;
+    const int K = A.K, O = A.O;
+    const int col0 = DUAL ? (nb * kF32Waves + wave) * 16 : (nb * kF32Waves + wave) * 32;
+    if (col0 >= O)
+        return;  // past the last column tile (waves share nothing: no barrier below)
+    F32Item it;
+    if (A.items) {
+        it = A.items[item];
+    } else {
+        it.a = 0;
+        it.r0 = item * 16 * MT;
+        it.nrow = min(16 * MT, A.nrows_all - it.r0);
+    }
+    const ExpertWork &ew = A.items ? A.ew[it.a] : A.ew1;
+    const int jbase = ew.row0 + it.r0;
+    // operand row pointers of this lane: MT input rows, two weight rows
+    const float4 *xr[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int r = min(mt * 16 + t, it.nrow - 1);  // rows past the item repeat the last
+        const int src = A.in_rows ? A.in_rows[jbase + r] : jbase + r;
+        xr[mt] = reinterpret_cast<const float4 *>(A.in + (size_t)src * K) + q;
+    }
+    const float4 *wr[2];
+    const int *wr8[2];  // I8: 4 codes of row t at K offset 4 q of each 16-wide block
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        const int row = DUAL ? col0 + t : col0 + 16 * m + t;
+        if constexpr (I8) {
+            const int8_t *w = static_cast<const int8_t *>(ew.w[A.mi]);
+            wr8[m] = reinterpret_cast<const int *>(w + (size_t)row * K) + q;
+        } else {
+            const float *w = static_cast<const float *>(ew.w[DUAL ? m : A.mi]);
+            wr[m] = reinterpret_cast<const float4 *>(w + (size_t)row * K) + q;
+        }
+    }
+    f4v acc[MT][2], tot[MT][2];  // tot: FOLD
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+        acc[mt][0] = acc[mt][1] = tot[mt][0] = tot[mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
+    const int nkb = K >> 4;  // 16-wide K blocks; a block is 4 float4 per row
+    float4 xa[2][MT], wb[2][2];
+    int wq[2][2];  // I8: raw codes
+    auto load = [&](int kb, int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+            xa[buf][mt] = xr[mt][4 * kb];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            if constexpr (I8)
+                wq[buf][m] = wr8[m][4 * kb];
+            else
+                wb[buf][m] = wr[m][4 * kb];
+        }
+    };
+    auto mma = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                float4 b;
+                if constexpr (I8) {
+                    const int v = wq[buf][m];
+                    b = float4{(float)(int8_t)(v & 0xff), (float)(int8_t)((v >> 8) & 0xff),
+                               (float)(int8_t)((v >> 16) & 0xff), (float)(int8_t)(v >> 24)};
+                } else {
+                    b = wb[buf][m];
+                }
+                const float4 a = xa[buf][mt];
+                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc[mt][m], 0, 0, 0);
+                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc[mt][m], 0, 0, 0);
+                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc[mt][m], 0, 0, 0);
+                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc[mt][m], 0, 0, 0);
+            }
+    };
+    // two blocks in flight: block kb + 1 loads while block kb multiplies (past the end:
+    // the last block again, never consumed)
+    load(0, 0);
+    for (int kb = 0; kb < nkb; kb += 2) {
+        load(min(kb + 1, nkb - 1), 1);
+        mma(0);
+        if (kb + 1 >= nkb)
+            break;
+        load(min(kb + 2, nkb - 1), 0);
+        mma(1);
+        if constexpr (FOLD)
+            if ((kb & 14) == 14)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) {
+                        tot[mt][m] += acc[mt][m];
+                        acc[mt][m] = f4v{0.f, 0.f, 0.f, 0.f};
+                    }
+    }
+    if constexpr (FOLD)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                acc[mt][m] += tot[mt][m];
+    // C[4 q + i][t] of row tile mt and column tile m
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = mt * 16 + 4 * q + i;
+            if (r >= it.nrow)
+                continue;
+            float *dst = A.out + (size_t)(jbase + r) * O;
+            if constexpr (DUAL) {
+                dst[col0 + t] = mf_act(A.act, acc[mt][0][i], acc[mt][1][i], A.act_a, A.act_b);
+            } else if constexpr (I8) {
+                const float *sc = static_cast<const float *>(ew.s[A.mi]);
+                dst[col0 + t] = acc[mt][0][i] * sc[col0 + t];
+                dst[col0 + 16 + t] = acc[mt][1][i] * sc[col0 + 16 + t];
+            } else {
+                dst[col0 + t] = acc[mt][0][i];
+                dst[col0 + 16 + t] = acc[mt][1][i];
+            }
+        }
+}
+
 bool f32mm_fits(bool dual, int K, int O) {
     return K >= 16 && K % 16 == 0 && O % (dual ? 16 : 32) == 0;
+}
+
+// Whether a wave of its own for each tile is the faster form: by K and the number of column
+// tiles of all items (32 columns; dual 16), from calls of 1 to 4096 rows and 32 to 163840
+// columns in both forms.  At few tiles it wins while K has no blocks for eight waves (f32 2048
+// x 64 at 16 rows 5.8 us with the split, 3.8 with a wave a tile); where the tiles are more
+// workgroups of eight waves than the chip holds, also beyond (f32 32768 x 512 at 16 rows 25 ->
+// 16, 65536 x 1024 91 -> 54, int8 24576 x 512 20 -> 15; against the blocks of 64 rows through
+// LDS, f32 16384 x 16 at 4096 rows 239 -> 47, int8 338 -> 75).  Between, the lines lie where the
+// split's gain at one row is no smaller than its loss at sixteen.  f32 K = 320 is there
+// because the blocks through LDS take K in pairs of 64.
+static bool f32_wave_fits(bool i8, int mt, int K, long long tiles, int rows) {
+    constexpr int kNever = 1 << 30;
+    struct Line {
+        int K, tiles;  // up to this K, from this many tiles
+    };
+    static const Line lines[2][3][6] = {
+        {{{128, 0}, {192, 224}, {384, 384}, {512, 768}, {768, 2048}, {1024, 1024}},
+         {{64, 0}, {128, 224}, {192, 384}, {512, 768}, {1024, 1024}, {kNever, kNever}},
+         {{64, 0}, {96, 1024}, {192, 1536}, {256, kNever}, {320, 4096}, {kNever, kNever}}},
+        {{{96, 0}, {128, 224}, {256, 384}, {512, 768}, {768, 1024}, {kNever, kNever}},
+         {{96, 384}, {128, 768}, {256, 1024}, {320, 2048}, {kNever, kNever}, {kNever, kNever}},
+         {{64, 1024}, {96, 1536}, {192, 2048}, {256, 4096}, {320, 3072}, {kNever, kNever}}},
+    };
+    for (const Line &l : lines[i8 ? 1 : 0][mt == 4 ? 2 : mt - 1])
+        if (K <= l.K)
+            if (l.tiles < kNever)
+                return tiles >= l.tiles;
+            else
+                break;
+    // any K: the rows' loads of a split's eight waves cost more than they hide (f32 65536 x
+    // 7168 at 16 rows 493 us with the split, 418)
+    return !i8 && mt <= 2 && K > 1024 && tiles >= 2048 && rows > 8 * mt;
 }
 
 hipError_t launch_f32mm(bool dual, int mt, const ExpertWork *ew, const void *items, int n_items,
@@ -424,6 +593,32 @@ hipError_t launch_f32mm(bool dual, int mt, const ExpertWork *ew, const void *ite
     if (n_items <= 0)
         return hipSuccess;
     a.n_items = n_items;
+    const long long tiles = (long long)n_items * (O / (dual ? 16 : 32));
+    if (!out2 && (!dual || K <= 512) && f32_wave_fits(i8, mt, K, tiles, nrows_all)) {
+        a.nbn = (O / (dual ? 16 : 32) + kF32Waves - 1) / kF32Waves;
+        const dim3 grid((unsigned)(n_items * a.nbn)), block(64 * kF32Waves);
+#define MVLLM_F32W(D, M, I, F) \
+    hipLaunchKernelGGL((k_f32mm_wave<D, M, I, F>), grid, block, 0, st, a)
+#define MVLLM_F32W_MT(D, I)                               \
+    do {                                                  \
+        if (mt == 1) MVLLM_F32W(D, 1, I, false);          \
+        else if (mt == 2) MVLLM_F32W(D, 2, I, false);     \
+        else MVLLM_F32W(D, 4, I, false);                  \
+    } while (0)
+        if (dual)
+            MVLLM_F32W_MT(true, false);
+        else if (i8)
+            MVLLM_F32W_MT(false, true);
+        else if (K > 512 && mt == 1)
+            MVLLM_F32W(false, 1, false, true);
+        else if (K > 512 && mt == 2)
+            MVLLM_F32W(false, 2, false, true);
+        else
+            MVLLM_F32W_MT(false, false);
+#undef MVLLM_F32W_MT
+#undef MVLLM_F32W
+        return hipGetLastError();
+    }
     // Blocks of 64 rows through LDS where they are more than a workgroup a CU (at 256 of them:
     // int8 1024 x 7168 at 512 rows 91 us against 82 of the rows' kernel, f32 91 against 88; at
     // 320, 2048 x 6144 at 300 rows, 128 against 144, int8 128 against 137).  Four weight tiles

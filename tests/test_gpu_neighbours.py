@@ -66,6 +66,8 @@ F32_CASES = [
     (4160, 3600, [2], 2, 2, 4.0, 25.0),             # 16-column dual tiles, 16 waves
     (96, 2064, [64, 64, 33], 70, 2, 4.0, 25.0),     # 64-row blocks, 4 weight tiles, ragged columns
     (1056, 2064, [130, 64, 40], 150, 1, 7.0, 0.0),  # 64-row blocks, 2 weight tiles, chains of 512
+    (64, 48, [20, 3, 0, 70], 90, 2, 4.0, 25.0),     # short K: a wave a tile, all row classes
+    (160, 6176, [16, 9], 20, 1, 7.0, 0.0),          # a wave a tile by the number of tiles
 ]
 
 
@@ -165,7 +167,10 @@ def test_router_workspace_shared(hip, T, D, E, k, shared):
                                        (0, 32, 16, 1), (0, 480, 1040, 17), (0, 7200, 4112, 16),
                                        (8, 160, 4160, 33), (8, 7200, 4096, 2), (8, 32, 80, 65),
                                        (0, 4128, 80, 129), (0, 4128, 16, 300), (0, 4128, 1040, 300),
-                                       (8, 4128, 144, 129), (8, 4128, 1040, 257)])
+                                       (8, 4128, 144, 129), (8, 4128, 1040, 257),
+                                       (0, 160, 64, 65), (0, 24576, 496, 3), (0, 24608, 272, 17),
+                                       (0, 32768, 528, 9), (0, 32768, 544, 17), (0, 32800, 96, 40),
+                                       (8, 160, 96, 16), (8, 12288, 96, 17), (8, 35872, 48, 33)])
 def test_linear(hip, orc, fmt, O, K, n):
     """fmt 8 (QuantMat's int8 rows, MVLLM_DENSE_BITS=8) at K3's latent shapes, with codes
     and scales from the reference's quantizer rule (row amax / 127, clamp +-127) and an
