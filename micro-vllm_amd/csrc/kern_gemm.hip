@@ -905,9 +905,15 @@ __global__ __launch_bounds__(256) void k_sum_splits(const f4v *part, f4u *y, siz
 // 32 and 64 rows), plus the launch that adds the sums and their bytes.  Per call with its
 // planes, unsplit -> split: int4 2048 x 6144 at 1 row 51 -> 15 us, at 100 rows 108 -> 27, at
 // 512 rows 111 -> 47; 7168 x 7168 at 61 rows 128 -> 33; 4096 x 4096 at 1024 rows stays whole
-// (256 workgroups, 82 us).
+// (256 workgroups, 82 us).  Up to 32 rows the weights' stream is the bound from some 160
+// workgroups on and splits add only their sums: MXFP4 65536 x 7168 at 16 rows 53 us split, 46
+// whole, 49152 x 4096 at 1 row 36 against 27, 40960 x 7168 41 against 44; a shorter K, whose
+// splits are the dearer part, from 160 of 16 rows and 128 of 32 (32768 x 2048 at 32 rows 28
+// against 22 us).
 int gemm_rows_splits(int mt, int nrows, int K, int O) {
     const long long tasks = (long long)((nrows + 16 * mt - 1) / (16 * mt)) * (O / 256);
+    if (mt <= 2 && tasks >= (K >= 4096 ? 161 : mt == 2 ? 128 : 160))
+        return 1;
     const int np = (K / kGemmBK + 1) / 2, slots = mt == 4 ? 256 : 512;
     const double pair_us = mt == 4 ? 8. : mt == 2 ? 5. : 3.6;
     const double sum_us = (double)nrows * O * 8 / 4e6;  // 4 TB/s, written and read

@@ -335,7 +335,11 @@ def test_linear_int8_rows_aligned_to_four_bytes(hip, orc):
 @pytest.mark.parametrize("fmt,O,K,n", [(4, 512, 7168, 1), (7, 256, 2304, 17), (4, 256, 2304, 100),
                                        (7, 512, 6144, 65), (4, 256, 2048, 16), (7, 256, 2048, 17),
                                        (4, 512, 1024, 32), (7, 256, 512, 64), (4, 256, 512, 65),
-                                       (4, 512, 512, -5), (7, 2304, 2304, -33)])
+                                       (4, 512, 512, -5), (7, 2304, 2304, -33),
+                                       # either side of the launches that stay whole
+                                       (7, 32512, 2304, 17), (7, 32768, 2304, 17),
+                                       (4, 40704, 2304, 3), (4, 40960, 2304, 3),
+                                       (7, 40960, 4096, 2), (7, 41216, 4096, 2)])
 def test_linear_splits_against_64_bits(hip, fmt, O, K, n):
     """K split over workgroups (whole and ragged ranges of step pairs) and the few-row launch on
     either side of its line; n < 0: y overwrites x.  Two bf16 terms are 2^-17 of each product, the
