@@ -308,6 +308,35 @@ __global__ __launch_bounds__(64 * W) void k_q_rows(QArgs A) {
 // end before lane q's 16 of it).
 bool q_rows_fits(int fmt, int K) { return (fmt == 4 || fmt == 7) && K >= 64 && K % 16 == 0; }
 
+// Weight tiles of 16 a wave holds and, with them, the workgroups of a launch.  Four tiles share
+// one split of x, two give more workgroups: 4 from 512 two-tile tasks on (2 per CU).
+static int q_rows_tiles(bool dual, int mt, long long n_items, int O) {
+    const long long t2 = n_items * ((O + (dual ? 15 : 31)) / (dual ? 16 : 32));
+    return mt == 1 && t2 >= 512 ? 4 : 2;
+}
+static long long q_rows_tasks(bool dual, long long n_items, int O, int nt) {
+    const int cols = (dual ? 8 : 16) * nt;
+    return n_items * ((O + cols - 1) / cols);
+}
+
+// A linear's few rows of a short K as one launch, where the planes, the GEMM and the sum of its
+// splits are three (7168 x 512 at 1 row 9.2 -> 6.0 us, at 32 rows 11.5 -> 6.8; 7168 x 1024 at
+// 16 rows 13.0 -> 9.9, 7168 x 2048 at 1 row 12.8 -> 11.0; equal at 2048 and 16 rows, behind past
+// it: 6144 at 1 row 14.6 -> 19.6).  A workgroup's time grows with K and a second one on a CU
+// runs after the first, so only launches of at most a workgroup a CU, two of a shorter K, are
+// ahead of the planes, whose GEMM reads wide matrices at the HBM's rate (32768 x 512 at 33
+// rows 37 us against 15, 65536 x 2048 at 1 row 49 against 22, 28672 x 512 at 1 row 11.9
+// against 9.3; MXFP4 16384 x 1024 at 16 rows 12.7 against 10.8, 10240 x 768 at 1 row 6.0
+// against 9.2, 7168 x 256 at 65 rows 13.7 against 10.6, at 64 rows 9.6).
+bool q_rows_linear(int K, int O, int n) {
+    const int mt = n <= 16 ? 1 : 2, nb = (n + 15) / 16, items = (n + 16 * mt - 1) / (16 * mt);
+    const bool wide = O > 8192;
+    const long long tasks = q_rows_tasks(false, items, O, q_rows_tiles(false, mt, items, O));
+    if (wide && (O > 16384 || K > 768 || (K < 512 && n > 8)))
+        return false;
+    return (long long)K * nb <= (wide ? 1024 : 2048) && tasks <= (K <= 768 ? 512 : 256);
+}
+
 hipError_t launch_q_rows(int fmt, bool dual, int mt, const ExpertWork *ew, const void *items,
                          int n_items, const ExpertWork *ew1, int nrows_all, const float *in,
                          const int *in_rows, float *out, int mi, int K, int O, int act,
@@ -333,16 +362,14 @@ hipError_t launch_q_rows(int fmt, bool dual, int mt, const ExpertWork *ew, const
         n_items = (nrows_all + 16 * mt - 1) / (16 * mt);
     if (n_items <= 0)
         return hipSuccess;
-    // Four tiles a wave share one split of x, two give more workgroups: 4 from 512 two-tile
-    // tasks on (2 per CU).  Four waves a workgroup: its start and end weigh less than a finer
-    // split of these short rows gains.  24 tokens, 32 int4 experts of 2112 x 704, per call: 55
-    // us (4 tiles), 61 (2 tiles), 74 and 91 us with eight waves; 100 tokens, 64 MXFP4 experts
-    // of 2080 x 1056: 144 / 168 / 181 / 222 us; one token, 4 of 2592 x 1248: 34 / 32 / 34 / 38.
-    const long long t2 = (long long)n_items * ((O + (dual ? 15 : 31)) / (dual ? 16 : 32));
-    const int nt = mt == 1 && t2 >= 512 ? 4 : 2, w = mt == 1 ? 4 : 8;
+    // Four waves a workgroup: its start and end weigh less than a finer split of these short
+    // rows gains.  24 tokens, 32 int4 experts of 2112 x 704, per call: 55 us (4 tiles), 61 (2
+    // tiles), 74 and 91 us with eight waves; 100 tokens, 64 MXFP4 experts of 2080 x 1056: 144 /
+    // 168 / 181 / 222 us; one token, 4 of 2592 x 1248: 34 / 32 / 34 / 38.
+    const int nt = q_rows_tiles(dual, mt, n_items, O), w = mt == 1 ? 4 : 8;
     const int cols = (dual ? 8 : 16) * nt;
     a.nbn = (O + cols - 1) / cols;
-    a.n_tasks = n_items * a.nbn;
+    a.n_tasks = (int)q_rows_tasks(dual, n_items, O, nt);
     const dim3 grid((unsigned)a.n_tasks), block((unsigned)(64 * w));
 #define MVLLM_Q(F, D, M, N, W_) hipLaunchKernelGGL((k_q_rows<F, D, M, N, W_>), grid, block, 0, st, a)
 #define MVLLM_Q_MT(F, D)                          \

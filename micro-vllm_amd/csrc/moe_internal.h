@@ -260,6 +260,8 @@ hipError_t launch_rmsnorm(const float *x, const float *w, float *y, int rows, in
 // Requires K % 16 == 0 and K >= 64 (q_rows_fits), 16-byte aligned input rows, 8-byte aligned weights
 // and 4-byte aligned int4 scales; any O.
 bool q_rows_fits(int fmt, int K);
+// Whether a dense linear of n rows is faster in this form than on the planes.
+bool q_rows_linear(int K, int O, int n);
 hipError_t launch_q_rows(int fmt, bool dual, int mt, const ExpertWork *ew, const void *items,
                          int n_items, const ExpertWork *ew1, int nrows_all, const float *in,
                          const int *in_rows, float *out, int mi, int K, int O, int act,

@@ -2562,13 +2562,10 @@ int mvllm_hip_linear_dev(int fmt, const void *w, const void *scales, int O, int 
     // sizes and addresses, on which its order against other calls must not.
     if (!order_after_previous(C, st))
         return 0;
-    // Few rows of a short K: one launch on the f32 rows themselves, where the planes, the GEMM
-    // and the sum of its splits are three (7168 x 512 at 1 row 9.2 -> 6.0 us, at 32 rows 11.5
-    // -> 6.8; 7168 x 1024 at 16 rows 13.0 -> 9.9, 7168 x 2048 at 1 row 12.8 -> 11.0; equal at
-    // 2048 and 16 rows, behind past it: 6144 at 1 row 14.6 -> 19.6).  Not where y overlaps x,
+    // Few rows of a short K: one launch on the f32 rows themselves.  Not where y overlaps x,
     // which the planes allow: its workgroups read x while others write y.
-    const bool apart = !overlap(x, (size_t)n * K * 4, y, (size_t)n * O * 4);
-    if ((long long)K * ((n + 15) / 16) <= 2048 && apart && aligned(x, 16)) {
+    if (q_rows_linear(K, O, n) && aligned(x, 16) &&
+        !overlap(x, (size_t)n * K * 4, y, (size_t)n * O * 4)) {
         HIP_TRY(launch_q_rows(fmt, false, n <= 16 ? 1 : 2, nullptr, nullptr, 0, &ew, n, x, nullptr,
                               y, 2, K, O, 0, 0.f, 0.f, st));
     } else {

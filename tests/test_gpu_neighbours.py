@@ -339,7 +339,11 @@ def test_linear_int8_rows_aligned_to_four_bytes(hip, orc):
                                        # either side of the launches that stay whole
                                        (7, 32512, 2304, 17), (7, 32768, 2304, 17),
                                        (4, 40704, 2304, 3), (4, 40960, 2304, 3),
-                                       (7, 40960, 4096, 2), (7, 41216, 4096, 2)])
+                                       (7, 40960, 4096, 2), (7, 41216, 4096, 2),
+                                       # either side of the few-row launch by its workgroups
+                                       (4, 8192, 256, 64), (4, 8192, 256, 65), (7, 4096, 256, 128),
+                                       (7, 16384, 768, 16), (7, 16640, 768, 1), (4, 8448, 256, 9),
+                                       (4, 8448, 256, 8), (4, 8448, 1024, 1), (7, 8448, 512, 32)])
 def test_linear_splits_against_64_bits(hip, fmt, O, K, n):
     """K split over workgroups (whole and ragged ranges of step pairs) and the few-row launch on
     either side of its line; n < 0: y overwrites x.  Two bf16 terms are 2^-17 of each product, the
