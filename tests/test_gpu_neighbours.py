@@ -396,6 +396,26 @@ def test_linears_wait_across_streams(hip, fmt):
         assert np.array_equal(g.view(np.uint32), e.view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt,O,K,n", [(4, 512, 2048, 1), (7, 512, 2048, 16), (4, 256, 512, 64),
+                                       (7, 256, 1024, 17), (7, 2048, 256, 33)])
+def test_few_row_linear_holds_f32(hip, fmt, O, K, n):
+    """The few-row launch takes x as three exact terms: against 64 bits on activations of all 24
+    bits its 2-norm error is that of at most 12 roundings a wave's sum and 3 between waves
+    (0.4 * 2^-24 each, the early ones less); two terms are off by 4e-6."""
+    errs = []
+    for seed in range(3):
+        rng = np.random.default_rng(seed + O + K + n + fmt)
+        x = rng.standard_normal((n, K)).astype(np.float32)
+        e = expert_arrays(rng, fmt, K, O)
+        y = torch.zeros((n, O), dtype=torch.float32, device="cuda")
+        hip.linear_dev(fmt, dev(e["gp"]), dev(e["gs"]), O, K, dev(x), n, y)
+        torch.cuda.synchronize()
+        exp = x.astype(np.float64) @ npref.dequant(fmt, e["gp"], e["gs"], K).astype(np.float64).T
+        errs.append(np.linalg.norm(y.cpu().numpy() - exp) / np.linalg.norm(exp))
+    say("  errors", errs)
+    assert np.mean(errs) < 1.2e-7
+
+
 def test_linear_splits_workspace(hip):
     """The 32 MiB of the K splits are allocated by the first call that splits, not by one that
     does not need them; a capture before that call runs unsplit, replays give the same bits

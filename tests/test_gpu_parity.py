@@ -368,6 +368,27 @@ def test_large_activations_small_scales(hip, orc, D, I):
 
 
 @pytest.mark.parametrize("fmt", [4, 7])
+@pytest.mark.parametrize("D,I", [(1568, 928), (560, 304)])
+def test_other_widths_hold_f32(hip, fmt, D, I):
+    """Experts of other widths against 64 bits, on activations of all 24 bits, in rows of both
+    row classes.  Products are exact and sums go by chains of 64, so the 2-norm error is that
+    of some dozen f32 roundings of a growing sum (0.4 * 2^-24 each, the early ones less):
+    1.5e-7 measured.  Two terms of x are off by 4e-6, one chain over a wave's K by 2.4e-7."""
+    say("f32 of other widths", fmt, D, I)
+    errs = []
+    for seed in range(3):
+        rng = np.random.default_rng(seed + D + fmt)
+        act, a, b = (2, 4.0, 25.0) if fmt == 7 else (0, 0.0, 0.0)
+        c = random_case(rng, fmt, D, I, [3, 17, 1], 21, act, a, b, zero_out=True)
+        c.rows[:] = np.arange(21, dtype=np.int32)
+        got = run_dev(hip, c, act, a, b)
+        exp = npref.moe_block64(*c.args(), act, a, b)
+        errs.append(np.linalg.norm(got - exp) / np.linalg.norm(exp))
+    say("  errors", errs)
+    assert np.mean(errs) < 1.7e-7
+
+
+@pytest.mark.parametrize("fmt", [4, 7])
 @pytest.mark.parametrize("path,D,I,gemm", [("elementwise", 250, 130, 0), ("widths", 256, 128, 0),
                                            ("decode", 512, 512, 2),
                                            ("gemm", 512, 256, 1)])
