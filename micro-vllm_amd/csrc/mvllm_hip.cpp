@@ -954,6 +954,12 @@ int finish_call(Ctx &C, hipStream_t st, int si) {
     return 1;
 }
 
+// Bytes of a drop-in call's activations from which their copy goes ahead while out is gathered;
+// below, one copy of both is the cheaper.  Per call, one copy against two, experts of 2048 x
+// 1024 resident: 1 row each 60 / 70 us, 8 rows (0.5 MB) 115 / 117, 16 rows 175 / 171, 128 rows
+// 1112 / 1007, 512 rows, staged, 5561 / 5026.
+constexpr size_t kHostSplitBytes = size_t(1) << 20;
+
 // One row class of the grouped GEMM: the 128-row blocks of MXFP4 experts in one-term
 // bf16 arithmetic take the wide-tile kernel when the shapes and alignment allow.
 hipError_t launch_gemm_cls(bool w16, int fmt, bool dual, int terms, int mt, const ExpertWork *ew,
@@ -1705,7 +1711,8 @@ int mvllm_hip_moe_block(int nb, int D, int Iinter, int fmt, int qgs, const void 
     P.ew.insert(P.ew.end(), miss.begin(), miss.end());
 
     // 3) the compact activation rows, then the destination rows of out (combine writes
-    // out_row = t), gathered into pinned memory: one H2D copy
+    // out_row = t), gathered into pinned memory: one H2D copy, or where the rows are many the
+    // activations' copy while out is gathered
     const size_t R = P.xrow.size(), T = P.out_row.size();
     const size_t xb = (R * D * 4 + 255) & ~size_t(255), ob = T * D * 4;
     HIP_TRY(C.hx.ensure(xb + ob));
@@ -1714,9 +1721,15 @@ int mvllm_hip_moe_block(int nb, int D, int Iinter, int fmt, int qgs, const void 
     float *dx = static_cast<float *>(C.Xc.p), *dout = dx + xb / 4;
     for (size_t j = 0; j < R; ++j)
         std::memcpy(hx + j * D, xg + (size_t)P.xrow[j] * D, (size_t)D * 4);
+    const bool split_copy = xb >= kHostSplitBytes;
+    if (split_copy)
+        HIP_TRY(hipMemcpyAsync(dx, hx, xb, hipMemcpyHostToDevice, st));
     for (size_t t = 0; t < T; ++t)
         std::memcpy(ho + t * D, out + (size_t)P.out_row[t] * D, (size_t)D * 4);
-    HIP_TRY(hipMemcpyAsync(dx, hx, xb + ob, hipMemcpyHostToDevice, st));
+    if (split_copy)
+        HIP_TRY(hipMemcpyAsync(dout, ho, ob, hipMemcpyHostToDevice, st));
+    else
+        HIP_TRY(hipMemcpyAsync(dx, hx, xb + ob, hipMemcpyHostToDevice, st));
     C.stats[3] += static_cast<double>((R + T) * D * 4);
     std::vector<int> dest_rows = P.out_row;
     for (size_t t = 0; t < T; ++t)

@@ -310,6 +310,26 @@ def test_moe_block_host_parity(hip, orc, case):
             assert np.array_equal(got[t], c.out[t])
 
 
+@pytest.mark.parametrize("nr", [[120], [140], [300, 1, 260]])
+def test_moe_block_host_large_rows(hip, nr):
+    """The drop-in on either side of 1 MiB of activations, from where they are copied while out
+    is gathered: equal bits to the device call on the same rows, rows of out that receive
+    nothing untouched."""
+    say("moe_block host, many rows", nr)
+    rng = np.random.default_rng(sum(nr))
+    c = random_case(rng, 7, 2048, 256, nr, 400, 2, 4.0, 25.0, (), 3)
+    got, touched = c.out.copy(), np.zeros(c.S, bool)
+    assert hip.moe_block(*c.args(got), 2, 4.0, 25.0) == 1
+    assert hip.set_option("combine_ordered", 1)
+    try:
+        exp = run_dev(hip, c, 2, 4.0, 25.0)
+    finally:
+        hip.set_option("combine_ordered", 0)
+    assert np.array_equal(got.view(np.uint32), exp.view(np.uint32))
+    touched[c.rows[(c.rows >= 0) & (c.rows < c.S)]] = True
+    assert np.array_equal(got[~touched], c.out[~touched])
+
+
 def test_validation_matches_reference(hip):
     say("validation")
     rng = np.random.default_rng(5)
