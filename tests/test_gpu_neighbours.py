@@ -396,6 +396,93 @@ def test_linears_wait_across_streams(hip, fmt):
         assert np.array_equal(g.view(np.uint32), e.view(np.uint32))
 
 
+def same_nonfinite(got, exp):
+    assert np.array_equal(np.isnan(got), np.isnan(exp))
+    assert np.array_equal(np.isinf(got), np.isinf(exp))
+    assert np.array_equal(np.sign(got[np.isinf(exp)]), np.sign(exp[np.isinf(exp)]))
+    return np.isfinite(exp)
+
+
+@pytest.mark.parametrize("fmt,O,K,n", [(0, 512, 2048, 5), (0, 2080, 1040, 200), (0, 96, 64, 40),
+                                       (8, 512, 2048, 5), (8, 2080, 1040, 300), (8, 96, 48, 20)])
+def test_linear_nonfinite_rows(hip, orc, fmt, O, K, n):
+    """Inf and NaN in x (and in f32 weights, int8 row scales) through the split of K, the
+    blocks through LDS (which pad K with zeros) and a wave a tile: they land where the
+    reference's sums put them, in their own rows and columns."""
+    rng = np.random.default_rng(O + K + n + fmt)
+    x = rng.standard_normal((n, K)).astype(np.float32)
+    x[1, K - 1], x[2, 0], x[n - 1, K // 2] = np.inf, np.nan, -np.inf
+    if fmt == 0:
+        w, sc = (rng.standard_normal((O, K)) * 0.05).astype(np.float32), None
+        w[3, K - 2], w[O - 1, 5] = np.nan, np.inf
+    else:
+        w = rng.integers(-127, 128, (O, K)).astype(np.int8)
+        w[5, K - 1] = 0  # 0 * inf
+        sc = rng.uniform(0.001, 0.01, O).astype(np.float32)
+        sc[7], sc[O - 1] = np.inf, np.nan
+    y = torch.zeros((n, O), dtype=torch.float32, device="cuda")
+    hip.linear_dev(fmt, dev(w), None if sc is None else dev(sc), O, K, dev(x), n, y)
+    torch.cuda.synchronize()
+    got, exp = y.cpu().numpy(), orc.matmul(fmt, x, w, sc)
+    assert np.isnan(exp).any() and np.isinf(exp).any()
+    fin = same_nonfinite(got, exp)
+    assert npref.rel_err(got[fin], exp[fin]) < TOL_F32
+
+
+@pytest.mark.parametrize("fmt", [4, 7])
+@pytest.mark.parametrize("O,K,n", [(512, 512, 20), (256, 1024, 7), (512, 7168, 3), (512, 2304, 40),
+                                   (256, 6144, 100)])
+def test_linear_nonfinite_scales(hip, orc, fmt, O, K, n):
+    """Non-finite int4 scales, ue8m0 bytes 0, 1, 254 and 255 and an infinite activation through
+    the few-row launch and through K splits, whose ranges form such sums again by themselves."""
+    rng = np.random.default_rng(O + K + n + fmt)
+    x = rng.standard_normal((n, K)).astype(np.float32)
+    x[n - 1, K - 3] = np.inf
+    e = expert_arrays(rng, fmt, K, O)
+    s = e["gs"]
+    if fmt == 4:
+        s[3, 0], s[O - 1, -1], s[40, s.shape[1] // 2] = np.inf, -np.inf, np.nan
+    else:
+        s[3, 0], s[O - 1, -1], s[40, s.shape[1] // 2], s[41, 1], s[42, 2] = 255, 255, 0, 1, 254
+    y = torch.zeros((n, O), dtype=torch.float32, device="cuda")
+    hip.linear_dev(fmt, dev(e["gp"]), dev(s), O, K, dev(x), n, y)
+    torch.cuda.synchronize()
+    got, exp = y.cpu().numpy(), orc.matmul(fmt, x, e["gp"], s)
+    assert not np.isfinite(exp).all()
+    fin = same_nonfinite(got, exp)
+    rest = np.abs(exp) < 1e30  # byte 254: products of 2^127 stand apart from the rest
+    assert npref.rel_err(got[fin & rest], exp[fin & rest]) < 1e-4
+
+
+@pytest.mark.parametrize("T,D,E,k", [(3, 2048, 384, 8), (5, 1024, 64, 64), (40, 7168, 512, 4),
+                                     (2, 64, 544, 6)])
+def test_router_nonfinite(hip, orc, T, D, E, k):
+    """A bias of -inf masks experts (they are picked last, by index), +inf forces them; an
+    infinite activation saturates the sigmoid; of a token of NaN activations the picks are
+    distinct experts."""
+    rng = np.random.default_rng(T + D + E)
+    x = rng.standard_normal((T, D)).astype(np.float32)
+    w = (rng.standard_normal((E, D)) / np.sqrt(D)).astype(np.float32)
+    bias = (rng.standard_normal(E) * 0.05).astype(np.float32)
+    bias[rng.permutation(E)[:E - min(k, E // 2)]] = -np.inf
+    bias[np.nonzero(np.isfinite(bias))[0][0]] = np.inf
+    x[0, 3], x[T - 1, 5] = np.inf, np.nan
+    f32 = dict(dtype=torch.float32, device="cuda")
+    scores, choice = torch.empty((T, E), **f32), torch.empty((T, E), **f32)
+    idx, wt = torch.empty((T, k), dtype=torch.int32, device="cuda"), torch.empty((T, k), **f32)
+    hip.router_dev(dev(x), dev(w), dev(bias), T, D, E, k, 2.5, scores, choice, idx, wt)
+    torch.cuda.synchronize()
+    gi, gw, mix = idx.cpu().numpy(), wt.cpu().numpy(), scores.cpu().numpy()
+    ei, ew = orc.route(x[:T - 1], w, bias, k, 2.5)
+    assert np.array_equal(np.sort(gi[:T - 1], axis=1), np.sort(ei, axis=1))
+    go, eo = np.argsort(gi[:T - 1], axis=1), np.argsort(ei, axis=1)
+    assert np.allclose(np.take_along_axis(gw[:T - 1], go, 1), np.take_along_axis(ew, eo, 1),
+                       rtol=1e-5, atol=1e-7)
+    assert np.isin(mix[0], (0.0, 1.0)).all() and np.isnan(mix[T - 1]).all()
+    last = gi[T - 1]
+    assert len(set(last)) == k and last.min() >= 0 and last.max() < E
+
+
 @pytest.mark.parametrize("fmt,O,K,n", [(4, 512, 2048, 1), (7, 512, 2048, 16), (4, 256, 512, 64),
                                        (7, 256, 1024, 17), (7, 2048, 256, 33)])
 def test_few_row_linear_holds_f32(hip, fmt, O, K, n):

@@ -576,6 +576,56 @@ def test_promote_hits_and_evict(hip, orc):
         hip.evict(0, int(e))
 
 
+@pytest.mark.parametrize("fmt", [4, 7])
+def test_widths_resident_and_staged(hip, orc, fmt):
+    """The drop-in at a width that is no multiple of 256, some experts promoted and some
+    staged, rows in both row classes on both sides (the gate/up launches of the resident part
+    run before the wait for the staged copies): against the oracle, and equal bits to the call
+    with every expert staged."""
+    say("widths, resident and staged", fmt)
+    rng = np.random.default_rng(70 + fmt)
+    D, I, layer = 2112, 704, 71
+    act, a, b = (2, 4.0, 25.0) if fmt == 7 else (1, 7.0, 0.0)
+    c = random_case(rng, fmt, D, I, [3, 20, 16, 0, 33, 1], 50, act, a, b, (), 2)
+    n, off = hip.expert_geom(fmt, D, I)
+    L, slots = hip.lib(), []
+    lists = [[] for _ in range(6)]  # g, u, d, gs, us, ds in the slots
+    for e in range(c.nb):
+        p = L.mvllm_hip_host_alloc(n)
+        assert p
+        slots.append(p)
+        for i, (arr, o) in enumerate(zip((c.g, c.u, c.d, c.gs, c.us, c.ds),
+                                         (off[0], off[2], off[4], off[1], off[3], off[5]))):
+            src = arr[e]
+            view = np.frombuffer((ctypes.c_uint8 * src.nbytes).from_address(p + int(o)),
+                                 src.dtype).reshape(src.shape)
+            view[:] = src
+            lists[i].append(view)
+    args = lambda out: (c.nb, D, I, fmt, *lists, c.xg, c.xoff, c.nr, c.rows, c.rw, out,  # noqa: E731
+                        c.S, act, a, b)
+    exp = oracle_out(orc, c, act, a, b)
+    try:
+        staged = c.out.copy()
+        assert hip.moe_block(*args(staged)) == 1
+        assert npref.rel_err(staged, exp) < TOL_F32
+        for e in (1, 2, 5):
+            hip.promote(slots[e], n, layer, e)
+        hip.stats_reset()
+        got = c.out.copy()
+        assert hip.moe_block(*args(got)) == 1
+        st = hip.stats()
+        assert st["resident_hits"] == 3 and st["misses"] == 2
+        assert npref.rel_err(got, exp) < TOL_F32
+        # the combine's order is the caller's experts', whichever part they are in
+        assert np.array_equal(got.view(np.uint32), staged.view(np.uint32))
+    finally:
+        for e in range(c.nb):
+            hip.evict(layer, e)
+        torch.cuda.synchronize()
+        for p in slots:
+            L.mvllm_hip_host_free(p)
+
+
 def test_two_streams_in_sequence(hip, orc):
     say("two streams")
     rng = np.random.default_rng(44)

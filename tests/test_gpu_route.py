@@ -151,9 +151,11 @@ def test_segments_arbitrary_ids(hip, orc, T, topk, E):
     check_segments(orc, idx, wt, got, E)
 
 
-def test_segments_caps_and_bad_ids(hip, orc):
+@pytest.mark.parametrize("T,topk,E", [(200, 4, 40), (300, 4, 40), (20, 4, 1100), (700, 3, 1500)])
+def test_segments_caps_and_bad_ids(hip, orc, T, topk, E):
+    """Short capacities and an id past the experts, in the one-workgroup form and in the four
+    launches (by the pairs, by the experts, by both)."""
     rng = np.random.default_rng(5)
-    T, topk, E = 200, 4, 40
     idx = rng.integers(0, E, size=(T, topk)).astype(np.int32)
     wt = rng.uniform(0.1, 1.0, size=(T, topk)).astype(np.float32)
     # union truncated to the 10 smallest ids, as the host union does
