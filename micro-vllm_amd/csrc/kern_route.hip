@@ -21,15 +21,12 @@
 
 namespace mvllm_hip {
 
-// a ranks before b: larger score first, lower index on ties (the reference comparator;
-// -0 and +0 tie).  Scores are not NaN (the reference's sort has no order for NaN).
-__device__ __forceinline__ bool rank_before(float va, int a, float vb, int b) {
-    return va == vb ? a < b : va > vb;
-}
-
 constexpr int kTopkWaves = 4;
 
-// A score as an unsigned key of the same order (-0 and +0 alike); 0 is kept for "taken".
+// A score as an unsigned key of the same order (-0 and +0 alike); 0 is kept for "taken".  The
+// reference's sort has no order for NaN; by key it has one, so that every round picks some
+// expert (a NaN that compared with nothing left lanes without one, and their -1 was read as an
+// index).
 __device__ __forceinline__ uint32_t rank_key(float v) {
     const uint32_t b = __float_as_uint(v + 0.f);  // -0 + 0 = +0
     return max(b ^ ((uint32_t)((int)b >> 31) | 0x80000000u), 1u);
@@ -137,25 +134,25 @@ __global__ __launch_bounds__(64 * kTopkWaves) void k_moe_topk(const float *choic
     } else {
         uint64_t taken = 0;  // bit s: element lane + 64 s is picked (n_exp <= 4096)
         for (int i = 0; i < k; ++i) {
-            float bv = 0.f;
+            uint32_t bk = 0;  // larger key first, lower index on ties (the reference comparator)
             int bi = -1;
             for (int s = 0; lane + 64 * s < n_exp; ++s) {
                 const int j = lane + 64 * s;
                 if ((taken >> s) & 1u)
                     continue;
-                const float v = row[j];
-                if (bi < 0 || rank_before(v, j, bv, bi)) {
-                    bv = v;
+                const uint32_t key = rank_key(row[j]);
+                if (key > bk) {
+                    bk = key;
                     bi = j;
                 }
             }
             // the order is total on the candidates, so any reduction tree finds the same one
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) {
-                const float ov = __shfl_xor(bv, off);
+                const uint32_t ok = __shfl_xor(bk, off);
                 const int oi = __shfl_xor(bi, off);
-                if (oi >= 0 && (bi < 0 || rank_before(ov, oi, bv, bi))) {
-                    bv = ov;
+                if (ok > bk || (ok == bk && ok && oi < bi)) {
+                    bk = ok;
                     bi = oi;
                 }
             }

@@ -455,7 +455,7 @@ def test_linear_nonfinite_scales(hip, orc, fmt, O, K, n):
 
 
 @pytest.mark.parametrize("T,D,E,k", [(3, 2048, 384, 8), (5, 1024, 64, 64), (40, 7168, 512, 4),
-                                     (2, 64, 544, 6)])
+                                     (2, 64, 544, 6), (3, 64, 1024, 64)])
 def test_router_nonfinite(hip, orc, T, D, E, k):
     """A bias of -inf masks experts (they are picked last, by index), +inf forces them; an
     infinite activation saturates the sigmoid; of a token of NaN activations the picks are
