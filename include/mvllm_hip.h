@@ -186,7 +186,8 @@ int mvllm_hip_moe_segments_dev(const int *idx, const float *wt, int n_tok, int t
                                int cap_experts, int cap_rows, int *counts, void *stream);
 
 /* Both in one call: mvllm_hip_moe_topk_dev, then mvllm_hip_moe_segments_dev of its
- * idx / wt (same arguments, same results; five launches). */
+ * idx / wt (same arguments, same results; two launches up to 1024 (token, slot) pairs and
+ * 1024 experts, five beyond). */
 int mvllm_hip_moe_route_dev(const float *choice, const float *mix, int n_tok, int n_exp, int k,
                             int *idx, float *wt, int *work, int *eids, int *xoff, int *nr,
                             int *rows, float *rw, int cap_experts, int cap_rows, int *counts,
