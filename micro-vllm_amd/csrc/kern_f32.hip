@@ -399,10 +399,13 @@ constexpr int kF32Waves = 4;
 
 // Short K, or more column tiles than the chip holds workgroups: a wave of its own for each tile
 // of 16 MT rows x 32 columns (dual: 16) over all of K.  The splits above then start eight waves
-// and meet in LDS for a few blocks each.  int8 codes come as 4 of each 16-wide block.  FOLD
-// (K > 512): each 256 of K sum in their own chain, which then adds to the total.
-template <bool DUAL, int MT, bool I8, bool FOLD>
-__global__ __launch_bounds__(64 * kF32Waves) void k_f32mm_wave(F32Args A) {
+// and meet in LDS for a few blocks each.  int8 codes come as 4 of each 16-wide block.  K sums in
+// P chains, by the block's parity (P = 2, as the two groups above) and by the matrix
+// instruction's step in it (P = 8, as eight waves), added in order at the end: as exact as the
+// split (f32 24576 x 512 1.5e-7 from 64 bits, one chain 4.0e-7).
+template <bool DUAL, int MT, bool I8, int P>
+__global__ __launch_bounds__(64 * kF32Waves)
+__attribute__((amdgpu_waves_per_eu(MT == 2 ? 2 : 1, 8))) void k_f32mm_wave(F32Args A) {
     static_assert(!(I8 && DUAL), "int8 rows: single projections only");
     const int item = blockIdx.x / A.nbn;
     const int nb = blockIdx.x - item * A.nbn;
@@ -443,10 +446,12 @@ __global__ __launch_bounds__(64 * kF32Waves) void k_f32mm_wave(F32Args A) {
             wr[m] = reinterpret_cast<const float4 *>(w + (size_t)row * K) + q;
         }
     }
-    f4v acc[MT][2], tot[MT][2];  // tot: FOLD
+    f4v acc[P][MT][2];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-        acc[mt][0] = acc[mt][1] = tot[mt][0] = tot[mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+            acc[p][mt][0] = acc[p][mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
     const int nkb = K >> 4;  // 16-wide K blocks; a block is 4 float4 per row
     float4 xa[2][MT], wb[2][2];
     int wq[2][2];  // I8: raw codes
@@ -476,10 +481,14 @@ __global__ __launch_bounds__(64 * kF32Waves) void k_f32mm_wave(F32Args A) {
                     b = wb[buf][m];
                 }
                 const float4 a = xa[buf][mt];
-                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc[mt][m], 0, 0, 0);
-                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc[mt][m], 0, 0, 0);
-                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc[mt][m], 0, 0, 0);
-                acc[mt][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc[mt][m], 0, 0, 0);
+                auto step = [&](float x, float w, int s) __attribute__((always_inline)) {
+                    f4v &c = acc[P == 8 ? 4 * buf + s : P == 2 ? buf : 0][mt][m];
+                    c = __builtin_amdgcn_mfma_f32_16x16x4f32(x, w, c, 0, 0, 0);
+                };
+                step(a.x, b.x, 0);
+                step(a.y, b.y, 1);
+                step(a.z, b.z, 2);
+                step(a.w, b.w, 3);
             }
     };
     // two blocks in flight: block kb + 1 loads while block kb multiplies (past the end:
@@ -492,22 +501,14 @@ __global__ __launch_bounds__(64 * kF32Waves) void k_f32mm_wave(F32Args A) {
             break;
         load(min(kb + 2, nkb - 1), 0);
         mma(1);
-        if constexpr (FOLD)
-            if ((kb & 14) == 14)
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int m = 0; m < 2; ++m) {
-                        tot[mt][m] += acc[mt][m];
-                        acc[mt][m] = f4v{0.f, 0.f, 0.f, 0.f};
-                    }
     }
-    if constexpr (FOLD)
+#pragma unroll
+    for (int p = 1; p < P; ++p)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int m = 0; m < 2; ++m)
-                acc[mt][m] += tot[mt][m];
+                acc[0][mt][m] += acc[p][mt][m];
     // C[4 q + i][t] of row tile mt and column tile m
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -518,14 +519,14 @@ __global__ __launch_bounds__(64 * kF32Waves) void k_f32mm_wave(F32Args A) {
                 continue;
             float *dst = A.out + (size_t)(jbase + r) * O;
             if constexpr (DUAL) {
-                dst[col0 + t] = mf_act(A.act, acc[mt][0][i], acc[mt][1][i], A.act_a, A.act_b);
+                dst[col0 + t] = mf_act(A.act, acc[0][mt][0][i], acc[0][mt][1][i], A.act_a, A.act_b);
             } else if constexpr (I8) {
                 const float *sc = static_cast<const float *>(ew.s[A.mi]);
-                dst[col0 + t] = acc[mt][0][i] * sc[col0 + t];
-                dst[col0 + 16 + t] = acc[mt][1][i] * sc[col0 + 16 + t];
+                dst[col0 + t] = acc[0][mt][0][i] * sc[col0 + t];
+                dst[col0 + 16 + t] = acc[0][mt][1][i] * sc[col0 + 16 + t];
             } else {
-                dst[col0 + t] = acc[mt][0][i];
-                dst[col0 + 16 + t] = acc[mt][1][i];
+                dst[col0 + t] = acc[0][mt][0][i];
+                dst[col0 + 16 + t] = acc[0][mt][1][i];
             }
         }
 }
@@ -537,34 +538,32 @@ bool f32mm_fits(bool dual, int K, int O) {
 // Whether a wave of its own for each tile is the faster form: by K and the number of column
 // tiles of all items (32 columns; dual 16), from calls of 1 to 4096 rows and 32 to 163840
 // columns in both forms.  At few tiles it wins while K has no blocks for eight waves (f32 2048
-// x 64 at 16 rows 5.8 us with the split, 3.8 with a wave a tile); where the tiles are more
+// x 64 at 16 rows 5.8 us with the split, 4.4 with a wave a tile); where the tiles are more
 // workgroups of eight waves than the chip holds, also beyond (f32 32768 x 512 at 16 rows 25 ->
-// 16, 65536 x 1024 91 -> 54, int8 24576 x 512 20 -> 15; against the blocks of 64 rows through
-// LDS, f32 16384 x 16 at 4096 rows 239 -> 47, int8 338 -> 75).  Between, the lines lie where the
-// split's gain at one row is no smaller than its loss at sixteen.  f32 K = 320 is there
-// because the blocks through LDS take K in pairs of 64.
+// 20, 65536 x 1024 92 -> 62, int8 163840 x 16 60 -> 9; against the blocks of 64 rows through
+// LDS, f32 16384 x 16 at 4096 rows 240 -> 51).  One chain of K is some 20 % faster still, but
+// 2.6 times as far from 64 bits.  Up to four rows the split stays ahead for longer: there the
+// tiles of a longer K count half.
 static bool f32_wave_fits(bool i8, int mt, int K, long long tiles, int rows) {
     constexpr int kNever = 1 << 30;
     struct Line {
         int K, tiles;  // up to this K, from this many tiles
     };
-    static const Line lines[2][3][6] = {
-        {{{128, 0}, {192, 224}, {384, 384}, {512, 768}, {768, 2048}, {1024, 1024}},
-         {{64, 0}, {128, 224}, {192, 384}, {512, 768}, {1024, 1024}, {kNever, kNever}},
-         {{64, 0}, {96, 1024}, {192, 1536}, {256, kNever}, {320, 4096}, {kNever, kNever}}},
-        {{{96, 0}, {128, 224}, {256, 384}, {512, 768}, {768, 1024}, {kNever, kNever}},
-         {{96, 384}, {128, 768}, {256, 1024}, {320, 2048}, {kNever, kNever}, {kNever, kNever}},
-         {{64, 1024}, {96, 1536}, {192, 2048}, {256, 4096}, {320, 3072}, {kNever, kNever}}},
+    static const Line lines[2][3][7] = {
+        {{{96, 0}, {128, 224}, {320, 384}, {384, 768}, {512, 1024}, {768, kNever}, {1024, 1024}},
+         {{64, 0}, {192, 384}, {256, 768}, {512, 1024}, {1024, 2048}, {kNever, kNever}},
+         {{32, 0}, {64, 640}, {96, 1536}, {128, 24576}, {192, 5120}, {kNever, kNever}}},
+        {{{64, 0}, {128, 224}, {256, 384}, {384, 768}, {512, 1024}, {kNever, kNever}},
+         {{96, 384}, {256, 1024}, {kNever, kNever}},
+         {{16, 640}, {32, 896}, {96, 1536}, {192, 5120}, {256, kNever}, {320, 6144},
+          {kNever, kNever}}},
     };
+    if (mt == 1 && rows <= 4 && K > (i8 ? 128 : 320))
+        tiles /= 2;
     for (const Line &l : lines[i8 ? 1 : 0][mt == 4 ? 2 : mt - 1])
         if (K <= l.K)
-            if (l.tiles < kNever)
-                return tiles >= l.tiles;
-            else
-                break;
-    // any K: the rows' loads of a split's eight waves cost more than they hide (f32 65536 x
-    // 7168 at 16 rows 493 us with the split, 418)
-    return !i8 && mt <= 2 && K > 1024 && tiles >= 2048 && rows > 8 * mt;
+            return tiles >= l.tiles;
+    return false;
 }
 
 hipError_t launch_f32mm(bool dual, int mt, const ExpertWork *ew, const void *items, int n_items,
@@ -597,25 +596,25 @@ hipError_t launch_f32mm(bool dual, int mt, const ExpertWork *ew, const void *ite
         return hipSuccess;
     a.n_items = n_items;
     const long long tiles = (long long)n_items * (O / (dual ? 16 : 32));
-    if (!out2 && (!dual || K <= 512) && f32_wave_fits(i8, mt, K, tiles, nrows_all)) {
+    if (!out2 && f32_wave_fits(i8, mt, K, tiles, nrows_all)) {
         a.nbn = (O / (dual ? 16 : 32) + kF32Waves - 1) / kF32Waves;
         const dim3 grid((unsigned)(n_items * a.nbn)), block(64 * kF32Waves);
-#define MVLLM_F32W(D, M, I, F) \
-    hipLaunchKernelGGL((k_f32mm_wave<D, M, I, F>), grid, block, 0, st, a)
+#define MVLLM_F32W(D, M, I, P) \
+    hipLaunchKernelGGL((k_f32mm_wave<D, M, I, P>), grid, block, 0, st, a)
 #define MVLLM_F32W_MT(D, I)                               \
     do {                                                  \
-        if (mt == 1) MVLLM_F32W(D, 1, I, false);          \
-        else if (mt == 2) MVLLM_F32W(D, 2, I, false);     \
-        else MVLLM_F32W(D, 4, I, false);                  \
+        if (mt == 1) MVLLM_F32W(D, 1, I, 8);              \
+        else if (mt == 2) MVLLM_F32W(D, 2, I, 8);         \
+        else MVLLM_F32W(D, 4, I, 2);                      \
     } while (0)
         if (dual)
             MVLLM_F32W_MT(true, false);
+        else if (K == 16 && mt == 4 && i8)  // one block: no second chain
+            MVLLM_F32W(false, 4, true, 1);
+        else if (K == 16 && mt == 4)
+            MVLLM_F32W(false, 4, false, 1);
         else if (i8)
             MVLLM_F32W_MT(false, true);
-        else if (K > 512 && mt == 1)
-            MVLLM_F32W(false, 1, false, true);
-        else if (K > 512 && mt == 2)
-            MVLLM_F32W(false, 2, false, true);
         else
             MVLLM_F32W_MT(false, false);
 #undef MVLLM_F32W_MT

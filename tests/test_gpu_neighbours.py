@@ -66,7 +66,8 @@ F32_CASES = [
     (4160, 3600, [2], 2, 2, 4.0, 25.0),             # 16-column dual tiles, 16 waves
     (96, 2064, [64, 64, 33], 70, 2, 4.0, 25.0),     # 64-row blocks, 4 weight tiles, ragged columns
     (1056, 2064, [130, 64, 40], 150, 1, 7.0, 0.0),  # 64-row blocks, 2 weight tiles, chains of 512
-    (64, 48, [20, 3, 0, 70], 90, 2, 4.0, 25.0),     # short K: a wave a tile, all row classes
+    (64, 48, [20, 3, 0, 70], 90, 2, 4.0, 25.0),     # short K: a wave a tile
+    (32, 32, [70, 33, 17, 1], 90, 1, 7.0, 0.0),     # the same, all row classes
     (160, 6176, [16, 9], 20, 1, 7.0, 0.0),          # a wave a tile by the number of tiles
 ]
 
@@ -168,9 +169,15 @@ def test_router_workspace_shared(hip, T, D, E, k, shared):
                                        (8, 160, 4160, 33), (8, 7200, 4096, 2), (8, 32, 80, 65),
                                        (0, 4128, 80, 129), (0, 4128, 16, 300), (0, 4128, 1040, 300),
                                        (8, 4128, 144, 129), (8, 4128, 1040, 257),
-                                       (0, 160, 64, 65), (0, 24576, 496, 3), (0, 24608, 272, 17),
-                                       (0, 32768, 528, 9), (0, 32768, 544, 17), (0, 32800, 96, 40),
-                                       (8, 160, 96, 16), (8, 12288, 96, 17), (8, 35872, 48, 33)])
+                                       # a wave a tile: ragged workgroups, odd numbers of
+                                       # blocks, either side of its lines
+                                       (0, 160, 64, 16), (0, 12320, 304, 5), (0, 12256, 304, 5),
+                                       (0, 32768, 496, 9), (0, 32800, 1008, 16), (0, 160, 64, 17),
+                                       (0, 24608, 240, 32), (0, 32768, 512, 20), (0, 160, 32, 65),
+                                       (0, 160, 16, 130), (0, 20512, 64, 40), (0, 49184, 80, 33),
+                                       (8, 160, 64, 16), (8, 12320, 240, 7), (8, 32800, 496, 5),
+                                       (8, 12288, 96, 17), (8, 32768, 240, 32), (8, 20512, 16, 40),
+                                       (8, 28704, 32, 33), (8, 49184, 96, 64)])
 def test_linear(hip, orc, fmt, O, K, n):
     """fmt 8 (QuantMat's int8 rows, MVLLM_DENSE_BITS=8) at K3's latent shapes, with codes
     and scales from the reference's quantizer rule (row amax / 127, clamp +-127) and an
@@ -403,8 +410,8 @@ def same_nonfinite(got, exp):
     return np.isfinite(exp)
 
 
-@pytest.mark.parametrize("fmt,O,K,n", [(0, 512, 2048, 5), (0, 2080, 1040, 200), (0, 96, 64, 40),
-                                       (8, 512, 2048, 5), (8, 2080, 1040, 300), (8, 96, 48, 20)])
+@pytest.mark.parametrize("fmt,O,K,n", [(0, 512, 2048, 5), (0, 2080, 1040, 200), (0, 96, 64, 20),
+                                       (8, 512, 2048, 5), (8, 2080, 1040, 300), (8, 96, 48, 12)])
 def test_linear_nonfinite_rows(hip, orc, fmt, O, K, n):
     """Inf and NaN in x (and in f32 weights, int8 row scales) through the split of K, the
     blocks through LDS (which pad K with zeros) and a wave a tile: they land where the
