@@ -250,8 +250,8 @@ int mvllm_hip_router_dev(const float *x, const float *w, const float *bias, int 
  * 2003-2006, 2074-2090).  fmt 0: f32 W [O][K] on the f32 matrix cores (K % 16, O % 32,
  * 16-byte aligned rows); fmt 4 / 7: W codes [O][K/2] with scales as in moe_block, the
  * input rows as two bf16 terms (2^-17 relative) on the bf16 matrix cores (K % 256,
- * O % 256); calls of few rows of a short K (K * ceil(n / 16) <= 2048 and O <= 16384 at
- * most), where x is 16-byte aligned and y does not overlap it, as three terms, exact;
+ * O % 256); calls of few rows of a short K (K * ceil(n / 16) <= 2048), where x is 16-byte
+ * aligned and y does not overlap it, as three terms, exact;
  * fmt 8: QuantMat's int8 rows W [O][K] with f32 row scales [O]
  * (quant::matmul_int8_row, src/quant/quant.cpp:255-268; MVLLM_DENSE_BITS=8), each code
  * exact in f32 on the f32 matrix cores and the row scale applied once to the finished

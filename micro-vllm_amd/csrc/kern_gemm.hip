@@ -946,14 +946,15 @@ hipError_t launch_gemm_rows(int fmt, int terms, int mt, const ExpertWork *ew1, i
     a.O = O;
     a.rcap = nrows;
     const int n_items = (nrows + 16 * mt - 1) / (16 * mt) * a.ks;
-    if (terms != 2)
-        return hipErrorInvalidValue;
     hipError_t e = hipErrorInvalidValue;
 #define MVLLM_ROWS(F)                                                                     \
-    e = mt == 1   ? launch_gemm_t<F, false, 2, 1, true>(a, n_items, st)                   \
-        : mt == 2 ? launch_gemm_t<F, false, 2, 2, true>(a, n_items, st)                   \
-        : mt == 4 ? launch_gemm_t<F, false, 2, 4, true>(a, n_items, st)                   \
-                  : hipErrorInvalidValue
+    e = terms == 3 && mt == 1   ? launch_gemm_t<F, false, 3, 1, true>(a, n_items, st)     \
+        : terms == 3 && mt == 2 ? launch_gemm_t<F, false, 3, 2, true>(a, n_items, st)     \
+        : terms != 2            ? hipErrorInvalidValue                                    \
+        : mt == 1               ? launch_gemm_t<F, false, 2, 1, true>(a, n_items, st)     \
+        : mt == 2               ? launch_gemm_t<F, false, 2, 2, true>(a, n_items, st)     \
+        : mt == 4               ? launch_gemm_t<F, false, 2, 4, true>(a, n_items, st)     \
+                                : hipErrorInvalidValue
     if (fmt == 4)
         MVLLM_ROWS(4);
     else if (fmt == 7)

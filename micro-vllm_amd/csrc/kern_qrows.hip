@@ -316,17 +316,17 @@ static long long q_rows_tasks(bool dual, long long n_items, int O, int nt) {
 // 16 rows 13.0 -> 9.9, 7168 x 2048 at 1 row 12.8 -> 11.0; equal at 2048 and 16 rows, behind past
 // it: 6144 at 1 row 14.6 -> 19.6).  A workgroup's time grows with K and a second one on a CU
 // runs after the first, so only launches of at most a workgroup a CU, two of a shorter K, are
-// ahead of the planes, whose GEMM reads wide matrices at the HBM's rate (32768 x 512 at 33
-// rows 37 us against 15, 65536 x 2048 at 1 row 49 against 22, 28672 x 512 at 1 row 11.9
-// against 9.3; MXFP4 16384 x 1024 at 16 rows 12.7 against 10.8, 10240 x 768 at 1 row 6.0
-// against 9.2, 7168 x 256 at 65 rows 13.7 against 10.6, at 64 rows 9.6).
+// ahead of the planes, which take three terms for such calls and whose GEMM reads wide
+// matrices at the HBM's rate (32768 x 512 at 33 rows 37 us against 14, 65536 x 2048 at 1 row 49
+// against 23, 28672 x 512 at 1 row 11.9 against 9.9; MXFP4 12288 x 1024 at 32 rows 19.6 against
+// 16.8, at 4 rows 10.8 against 12.2, 7168 x 256 at 100 rows 17.8 against 9.6).
 bool q_rows_linear(int K, int O, int n) {
     const int mt = n <= 16 ? 1 : 2, nb = (n + 15) / 16, items = (n + 16 * mt - 1) / (16 * mt);
     const bool wide = O > 8192;
     const long long tasks = q_rows_tasks(false, items, O, q_rows_tiles(false, mt, items, O));
-    if (wide && (O > 16384 || K > 768 || (K < 512 && n > 8)))
+    if (wide && (O > 16384 || K > 1024 || (K == 1024 && n > 8)))
         return false;
-    return (long long)K * nb <= (wide ? 1024 : 2048) && tasks <= (K <= 768 ? 512 : 256);
+    return (long long)K * nb <= (wide ? 1536 : 2048) && tasks <= (wide || K <= 768 ? 512 : 256);
 }
 
 hipError_t launch_q_rows(int fmt, bool dual, int mt, const ExpertWork *ew, const void *items,

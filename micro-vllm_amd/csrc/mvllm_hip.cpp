@@ -2568,23 +2568,27 @@ int mvllm_hip_linear_dev(int fmt, const void *w, const void *scales, int O, int 
     }
     ew.w[2] = w;
     ew.s[2] = scales;
-    const int terms = 2;
-    HIP_TRY(C.Lp.ensure((size_t)terms * 2 * n * K));
+    // Few rows of a short K: x as three terms, exact.  In one launch on the f32 rows themselves
+    // where that is ahead of the planes; not where y overlaps x, which the planes allow: its
+    // workgroups read x while others write y.
+    const bool three = (long long)K * ((n + 15) / 16) <= 2048 && aligned(x, 16) &&
+                       !overlap(x, (size_t)n * K * 4, y, (size_t)n * O * 4);
+    const bool few = three && q_rows_linear(K, O, n);
+    const int terms = three ? 3 : 2;
+    HIP_TRY(C.Lp.ensure((size_t)(few ? 2 : terms) * 2 * n * K));
     // A call on another stream than the previous one waits for it, as the block entry points'
     // do: the planes buffer is shared by every call, and the form a call takes depends on its
     // sizes and addresses, on which its order against other calls must not.
     if (!order_after_previous(C, st))
         return 0;
-    // Few rows of a short K: one launch on the f32 rows themselves.  Not where y overlaps x,
-    // which the planes allow: its workgroups read x while others write y.
-    if (q_rows_linear(K, O, n) && aligned(x, 16) &&
-        !overlap(x, (size_t)n * K * 4, y, (size_t)n * O * 4)) {
+    if (few) {
         HIP_TRY(launch_q_rows(fmt, false, n <= 16 ? 1 : 2, nullptr, nullptr, 0, &ew, n, x, nullptr,
                               y, 2, K, O, 0, 0.f, 0.f, st));
     } else {
-        // the input rows as two bf16 terms (2^-17 relative), then the grouped GEMM
+        // the input rows as bf16 terms, then the grouped GEMM (three terms of 64 rows do not fit
+        // its LDS: such calls take blocks of 32)
         HIP_TRY(launch_prep_planes(fmt, terms, x, nullptr, n, K, n, C.Lp.p, st));
-        const int mt = n <= 16 ? 1 : n <= 32 ? 2 : 4;
+        const int mt = n <= 16 ? 1 : n <= 32 || three ? 2 : 4;
         HIP_TRY(launch_gemm_rows(fmt, terms, mt, &ew, n, C.Lp.p, y,
                                  gemm_rows_splits(mt, n, K, O) > 1 ? splits_buffer(C, st) : nullptr,
                                  K, O, st));

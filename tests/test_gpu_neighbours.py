@@ -349,8 +349,8 @@ def test_linear_int8_rows_aligned_to_four_bytes(hip, orc):
                                        (7, 40960, 4096, 2), (7, 41216, 4096, 2),
                                        # either side of the few-row launch by its workgroups
                                        (4, 8192, 256, 64), (4, 8192, 256, 65), (7, 4096, 256, 128),
-                                       (7, 16384, 768, 16), (7, 16640, 768, 1), (4, 8448, 256, 9),
-                                       (4, 8448, 256, 8), (4, 8448, 1024, 1), (7, 8448, 512, 32)])
+                                       (7, 16384, 768, 32), (7, 16640, 768, 1), (4, 8448, 256, 48),
+                                       (4, 8448, 1024, 8), (7, 8448, 1024, 9), (7, 8448, 512, 49)])
 def test_linear_splits_against_64_bits(hip, fmt, O, K, n):
     """K split over workgroups (whole and ragged ranges of step pairs) and the few-row launch on
     either side of its line; n < 0: y overwrites x.  Two bf16 terms are 2^-17 of each product, the
@@ -491,11 +491,16 @@ def test_router_nonfinite(hip, orc, T, D, E, k):
 
 
 @pytest.mark.parametrize("fmt,O,K,n", [(4, 512, 2048, 1), (7, 512, 2048, 16), (4, 256, 512, 64),
-                                       (7, 256, 1024, 17), (7, 2048, 256, 33)])
+                                       (7, 256, 1024, 17), (7, 2048, 256, 33),
+                                       # on the planes
+                                       (4, 16640, 768, 1), (7, 8448, 1024, 16), (4, 8448, 2048, 16),
+                                       (7, 7168, 256, 65), (4, 16640, 512, 40), (7, 10240, 1024, 32)])
 def test_few_row_linear_holds_f32(hip, fmt, O, K, n):
-    """The few-row launch takes x as three exact terms: against 64 bits on activations of all 24
-    bits its 2-norm error is that of at most 12 roundings a wave's sum and 3 between waves
-    (0.4 * 2^-24 each, the early ones less); two terms are off by 4e-6."""
+    """Few rows of a short K enter as three exact terms, in one launch or, of many columns, on
+    planes: against 64 bits on activations of all 24 bits the 2-norm error is that of at most 12
+    roundings a wave's sum and 3 between waves (0.4 * 2^-24 each, the early ones less), or of
+    the planes' one chain of up to 32 groups or 192 products (1e-7 and 3e-7 measured); two terms
+    are off by 4e-6."""
     errs = []
     for seed in range(3):
         rng = np.random.default_rng(seed + O + K + n + fmt)
@@ -507,7 +512,7 @@ def test_few_row_linear_holds_f32(hip, fmt, O, K, n):
         exp = x.astype(np.float64) @ npref.dequant(fmt, e["gp"], e["gs"], K).astype(np.float64).T
         errs.append(np.linalg.norm(y.cpu().numpy() - exp) / np.linalg.norm(exp))
     say("  errors", errs)
-    assert np.mean(errs) < 1.2e-7
+    assert np.mean(errs) < (1.2e-7 if O <= 2048 else 5e-7)
 
 
 def test_linear_splits_workspace(hip):
