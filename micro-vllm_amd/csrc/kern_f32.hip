@@ -542,8 +542,10 @@ bool f32mm_fits(bool dual, int K, int O) {
 // workgroups of eight waves than the chip holds, also beyond (f32 32768 x 512 at 16 rows 25 ->
 // 20, 65536 x 1024 92 -> 62, int8 163840 x 16 60 -> 9; against the blocks of 64 rows through
 // LDS, f32 16384 x 16 at 4096 rows 240 -> 51).  One chain of K is some 20 % faster still, but
-// 2.6 times as far from 64 bits.  Up to four rows the split stays ahead for longer: there the
-// tiles of a longer K count half.
+// 2.6 times as far from 64 bits.  The lines weigh single
+// matrices: small experts of 17 to 32 rows take up to 0.7 us more than with the split (eight of
+// 20 rows, 32 x 96 16.5 -> 17.2 us, 64 x 64 17.7 -> 18.0).  Up to four rows the split stays
+// ahead for longer: there the tiles of a longer K count half.
 static bool f32_wave_fits(bool i8, int mt, int K, long long tiles, int rows) {
     constexpr int kNever = 1 << 30;
     struct Line {

@@ -304,10 +304,21 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
         }
     };
 
-    f4v acc[MT][2];
+    // Three terms hold all 24 bits of x, which one chain over K would lose again: group g of each
+    // step has a sum of its own, accs[g], and the four are added in pairs at the end.  From 64
+    // bits at 65536 x 512 and 33 rows: MXFP4 2.1e-7 with one chain, 6e-8 so, int4 1.2e-7 and
+    // 7e-8, as near as the few-row launch, for up to 0.7 us (25.1 -> 25.6, 22.6 -> 23.3 us).
+    constexpr int NA = TERMS == 3 ? 4 : 1;
+    f4v accs[NA][MT][2];
+    auto &acc = accs[0];
+    auto clear = [&] __attribute__((always_inline)) () {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-        acc[mt][0] = acc[mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                accs[a][mt][0] = accs[a][mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
+    };
+    clear();
     const int src4 = 4 * (4 * t + q);  // ds_bpermute address of lane 4 t + q
 
 
@@ -401,14 +412,17 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
                 } else {
                     read_a(mt, a);
                 }
-                if constexpr (FMT == 4) {
-                    // each 64-wide group is its own chain over n - 8, then one f32 FMA
-                    // applies the group's scale
+                auto &sum = accs[NA == 4 ? g : 0];
+                if constexpr (FMT == 4 || TERMS == 3) {
+                    // int4: each 64-wide group is its own chain over n - 8, then one f32 FMA
+                    // applies the group's scale.  Three terms of either format: such a chain,
+                    // the lowest term first, so that few roundings are the size of the sum
 #pragma unroll
                     for (int m = 0; m < 2; ++m) {
                         f4v c = f4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                        for (int tm = 0; tm < TERMS; ++tm) {
+                        for (int i = 0; i < TERMS; ++i) {
+                            const int tm = TERMS == 3 ? 2 - i : i;
                             bf16x8 b0 = bf[m][0], b1 = bf[m][1];
                             if (EXACT && tm > 0 && spec[m])
                                 b0 = b1 = bf16x8{};
@@ -417,11 +431,12 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
                         }
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
-                            acc[mt][m][i] = EXACT && spec[m] ? acc[mt][m][i] + c[i]
-                                                             : fmaf(sg[m], c[i], acc[mt][m][i]);
+                            sum[mt][m][i] = FMT == 7 || (EXACT && spec[m])
+                                                ? sum[mt][m][i] + c[i]
+                                                : fmaf(sg[m], c[i], sum[mt][m][i]);
                         // keep the scaling here: sunk below the next step's loads, it
                         // drags a wait for those loads in with it
-                        asm volatile("" : "+v"(acc[mt][m]));
+                        asm volatile("" : "+v"(sum[mt][m]));
                     }
                 } else {
 #pragma unroll
@@ -737,11 +752,16 @@ __attribute__((amdgpu_waves_per_eu(MT == 2 && TERMS == 1 ? 4 : 1, 8))) void k_ge
     // the common pass.)
     if (__syncthreads_or((int)exc)) {
         exc = 0;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-            acc[mt][0] = acc[mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
+        clear();
         prologue();
         k_loop(std::true_type{});
+    }
+    if constexpr (NA == 4) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                acc[mt][m] = (accs[0][mt][m] + accs[1][mt][m]) + (accs[2][mt][m] + accs[3][mt][m]);
     }
     epilogue(cur);
 }

@@ -319,7 +319,7 @@ static long long q_rows_tasks(bool dual, long long n_items, int O, int nt) {
 // ahead of the planes, which take three terms for such calls and whose GEMM reads wide
 // matrices at the HBM's rate (32768 x 512 at 33 rows 37 us against 14, 65536 x 2048 at 1 row 49
 // against 23, 28672 x 512 at 1 row 11.9 against 9.9; MXFP4 12288 x 1024 at 32 rows 19.6 against
-// 16.8, at 4 rows 10.8 against 12.2, 7168 x 256 at 100 rows 17.8 against 9.6).
+// 17.2, at 4 rows 10.8 against 12.2, 7168 x 256 at 100 rows 17.8 against 9.9).
 bool q_rows_linear(int K, int O, int n) {
     const int mt = n <= 16 ? 1 : 2, nb = (n + 15) / 16, items = (n + 16 * mt - 1) / (16 * mt);
     const bool wide = O > 8192;

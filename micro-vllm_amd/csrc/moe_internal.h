@@ -220,9 +220,8 @@ hipError_t launch_gemm_wide(bool dual, const ExpertWork *ew, const void *items, 
                             const int *n_items_dev);
 // One matrix (w[2], s[2] of *ew1) over input rows [0, nrows) of the planes, in items of
 // 16 * mt rows computed in the kernel (a dense linear): out [nrows][O] f32; two terms, or three
-// with mt 1 or 2.  Launches of few
-// workgroups split K (gemm_rows_splits); the splits' sums go to part (kGemmRowsPart bytes;
-// null: no splits) and are added in order.
+// with mt 1 or 2.  Launches of few workgroups split K (gemm_rows_splits); the splits' sums go to
+// part (kGemmRowsPart bytes; null: no splits) and are added in order.
 constexpr size_t kGemmRowsPart = size_t(32) << 20;
 int gemm_rows_splits(int mt, int nrows, int K, int O);
 hipError_t launch_gemm_rows(int fmt, int terms, int mt, const ExpertWork *ew1, int nrows,

@@ -393,7 +393,8 @@ def test_other_widths_hold_f32(hip, fmt, D, I):
     """Experts of other widths against 64 bits, on activations of all 24 bits, in rows of both
     row classes.  Products are exact and sums go by chains of 64, so the 2-norm error is that
     of some dozen f32 roundings of a growing sum (0.4 * 2^-24 each, the early ones less):
-    1.5e-7 measured.  Two terms of x are off by 4e-6, one chain over a wave's K by 2.4e-7."""
+    1.5e-7 measured.  Two terms of x are off by 2.5e-6 in one projection, one chain over a
+    wave's K by 2.4e-7."""
     say("f32 of other widths", fmt, D, I)
     errs = []
     for seed in range(3):
